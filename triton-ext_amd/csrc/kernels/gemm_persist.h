@@ -9,11 +9,23 @@
 // loaded while the current one finishes and no tile pays a pipeline fill.
 //
 // Layout per workgroup: 4 wavefronts (one per SIMD) in a 2 x 2 grid, each
-// owning a BT / 2 square block of the tile; its accumulator blocks of 32 x 32
-// (BT = 256: 16 blocks, 256 registers) live in AGPRs.  Against the
-// 8-wavefront tile this reads a
-// third less from LDS per MFMA (1 KiB instead of 1.5), which the power-
+// owning a BT / 2 square block of the tile; its accumulator blocks of 16 x 16
+// (BT = 256: 64 blocks, 256 registers) live in AGPRs.  Against the
+// 8-wavefront tile this reads a third less from LDS per MFMA, which the power-
 // limited clock turns into speed.
+//
+// MFMA shape: 16x16x32 (16-bit) and 16x16x128 (fp8), not 32x32x16 / 32x32x64.
+// The large products are bound by the clock the power limit leaves, and the
+// 16 x 16 forms, which read and write a quarter of the accumulator per
+// instruction and sum twice the K, do the same work on less: register-only
+// loops on N(0,1) operands sustain 2025 against 1765 TFLOP/s (bf16) and 4360
+// against 3970 (fp8).  In this kernel (32 x 32 -> 16 x 16, same box): fp16
+// 4096^3 row-major B 110 -> 107 us (clock 1.75 -> 2.00 GHz, MFMA busy 64 ->
+// 60%), bf16 8192^3 764 -> 721 us, 2048^3 (BT = 128) 22.8 -> 21.6 us, fp8
+// 8192^3 371 -> 359 us.  Without the LDS-DMA stream (timing only) these take
+// 93, 628, 19.5 and 300 us: what binds them now is that stream's power and
+// its delivery, not MFMA issue (staggering reads and loads, or forcing the
+// accumulators in place, moves nothing beyond 1%).
 //
 // The K loop is that of gemm_fast_tile_at (ring of 5 LDS slots of BT x 128 bytes,
 // B of step s+2 and A of step s+3 loaded during the second half of step s,
@@ -50,21 +62,55 @@ namespace txg {
 namespace persist {
 constexpr int kWaves = 4;
 
-// Chunk swizzle of a K-major B slot (row-major K x N operand), by K row mod
-// 4, for K rows of krb bytes: 256 or more, (0, 6, 12, 10); 128 (8 chunks,
-// two rows per 256 bytes of banks), (0, 2, 4, 6).
-__device__ __forceinline__ constexpr int kn_swz(int rho, int krb) {
-  return krb >= 256 ? ((rho << 1) ^ (rho << 2)) & 14 : rho << 1;
+// Chunk swizzle of a K-major B slot (row-major K x N operand) for K row k, by
+// k mod 4 and bit 3 of k, for K rows of krb bytes: 256 or more, (0, 6, 12, 10)
+// and 2 more (XOR) in the second 8 rows of 16; 128 (8 chunks, two rows per
+// 256 bytes of banks), (0, 2, 4, 6), likewise.
+__device__ __forceinline__ constexpr int kn_swz(int k, int krb) {
+  const int rho = k & 3, hi = ((k >> 3) & 1) << 1;
+  return (krb >= 256 ? ((rho << 1) ^ (rho << 2)) & 14 : rho << 1) ^ hi;
 }
 
 // s_waitcnt lgkmcnt(N) that the two fragments depend on (their values come
 // from LDS reads issued in inline asm, which the compiler does not wait for).
 template <int N>
-__device__ __forceinline__ void lgkm_wait_tie(txd::i32x4 &x, txd::i32x4 &y) {
-  asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(x), "+v"(y) : "n"(N));
+__device__ __forceinline__ void lgkm_wait_tie(txd::i32x4 &x) {
+  asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(x) : "n"(N));
 }
 // The same dependency on a wait already made (the barrier's).
-__device__ __forceinline__ void tie(txd::i32x4 &x, txd::i32x4 &y) { asm volatile("" : "+v"(x), "+v"(y)); }
+__device__ __forceinline__ void tie(txd::i32x4 &x) { asm volatile("" : "+v"(x)); }
+
+// One 16 x 16 block product: 64 bytes of K of 16-bit operands (a 16-byte
+// piece per lane), or the 128 bytes of a whole step of fp8 (two).
+template <class C>
+__device__ __forceinline__ void mfma16(txd::f32x4 &acc, const txd::i32x4 (&b)[2], const txd::i32x4 (&a)[2], int h) {
+  if constexpr (C::FP8) {
+    const i32x8 vb = __builtin_shufflevector(b[0], b[1], 0, 1, 2, 3, 4, 5, 6, 7);
+    const i32x8 va = __builtin_shufflevector(a[0], a[1], 0, 1, 2, 3, 4, 5, 6, 7);
+    acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(vb, va, acc, F8Code<C::EL_B_>::v, F8Code<C::EL_A_>::v, 0, 0,
+                                                           0, 0);
+  } else if constexpr (C::F16) {
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(txd::f16x8, b[h]),
+                                                 __builtin_bit_cast(txd::f16x8, a[h]), acc, 0, 0, 0);
+  } else {
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(txd::bf16x8, b[h]),
+                                                  __builtin_bit_cast(txd::bf16x8, a[h]), acc, 0, 0, 0);
+  }
+}
+
+// fast::ktail_clear for this tile's fragments: lane l holds chunk 4h + l / 16
+// of the step in piece h.
+template <int NF>
+__device__ __forceinline__ void ktail_clear(txd::i32x4 (&fr)[NF][2], int h, int g, const fast::KTail &t) {
+  const bool hit = 4 * h + g == t.cp;
+  int m[4];
+#pragma unroll
+  for (int d = 0; d < 4; ++d) m[d] = hit ? int(t.keep[d]) : -1;
+#pragma unroll
+  for (int f = 0; f < NF; ++f)
+#pragma unroll
+    for (int d = 0; d < 4; ++d) fr[f][h][d] &= m[d];
+}
 
 // Buffer resource for rows r0 .. r0 + BT - 1 of an operand with `rows` rows of
 // `ld_b` bytes, K step bytes kb_end: rows past the operand's end are outside
@@ -101,8 +147,10 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
   static_assert(!BKN || (!C::FP8 && !GROUPED && !KTAIL), "row-major B: 16-bit operands, whole K steps");
   static_assert(BT == 256 || BT == 128 || BT == 64, "tile 256, 128 or 64 square");
   constexpr int NW = persist::kWaves;
-  constexpr int TM = BT / 2, TN = BT / 2, FM = TM / 32, FN = TN / 32;
-  constexpr int NM = FM * FN, NF = FM + FN, NR = 2 * NF;
+  constexpr int TM = BT / 2, TN = BT / 2, FM = TM / 16, FN = TN / 16;
+  // MFMAs of a K step's half (16-bit: K half h; fp8: half of the columns)
+  constexpr int NM = C::FP8 ? FM * FN / 2 : FM * FN, NF = FM + FN, NR = NF;
+  static_assert(!C::FP8 || BT == 256, "fp8: the 256 x 256 tile");
   constexpr int SB = BT * kStep;  // one operand of one K step
   constexpr int BLKA = SB / 1024 / NW, BLKB = BLKA, ND = BLKA + BLKB;
   constexpr int RW = NM >= 2 ? NM / 2 : 1;
@@ -132,19 +180,26 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
   // block j adds 8 j rows, and the K step, in the scalar offset.
   const uint32_t kch[2] = {16u * uint32_t((lane & 7) ^ ((lane >> 4) & 7)),
                            16u * uint32_t((lane & 7) ^ ((4 + (lane >> 4)) & 7))};
-  uint32_t vo[2][2];
+  // BKN block j: K rows RPB (BLKB wave + j) .. + RPB - 1 of the step, lane p
+  // filling chunk position p mod CPR of row + p / CPR.  The swizzle goes by
+  // the row's low two bits and bit 3, so block j shares the lane offsets of
+  // block kn_rep(j), kept at kn_var(j).
+  constexpr auto kn_rep = [](int j) constexpr { return BT == 256 ? (j & 1) + 4 * (j >> 2) : BT == 128 ? j & ~1 : j; };
+  constexpr auto kn_var = [](int j) constexpr { return BT == 256 ? (j & 1) + 2 * (j >> 2) : BT == 128 ? j >> 1 : j; };
+  constexpr int NVB = BKN && BT == 256 ? 4 : 2;
+  uint32_t vo[2][NVB];
 #pragma unroll
-  for (int e = 0; e < 2; ++e) {
-    vo[0][e] = uint32_t(8 * (BLKA * wave + e) + (lane >> 3)) * lda_b + kch[e];
-    if constexpr (BKN) {
-      // block j: K rows RPB (BLKB wave + j) .. + RPB - 1 of the step, lane p
-      // filling chunk position p mod CPR of row + p / CPR (row mod 4
-      // depends on the block's parity only)
-      const int kr = RPB * (BLKB * wave + e) + lane / CPR;
-      vo[1][e] = uint32_t(kr) * ldb_b + 16u * uint32_t((lane % CPR) ^ persist::kn_swz(kr & 3, KRB));
-    } else {
-      vo[1][e] = uint32_t(8 * (BLKB * wave + e) + (lane >> 3)) * ldb_b + kch[e];
+  for (int e = 0; e < 2; ++e) vo[0][e] = uint32_t(8 * (BLKA * wave + e) + (lane >> 3)) * lda_b + kch[e];
+  if constexpr (BKN) {
+#pragma unroll
+    for (int j = 0; j < BLKB; ++j) {
+      const int kr = RPB * (BLKB * wave + j) + lane / CPR;
+      if (j == kn_rep(j))
+        vo[1][kn_var(j)] = uint32_t(kr) * ldb_b + 16u * uint32_t((lane % CPR) ^ persist::kn_swz(kr, KRB));
     }
+  } else {
+#pragma unroll
+    for (int e = 0; e < 2; ++e) vo[1][e] = uint32_t(8 * (BLKB * wave + e) + (lane >> 3)) * ldb_b + kch[e];
   }
   const uint32_t ld8[2] = {8u * lda_b, (BKN ? uint32_t(RPB) : 8u) * ldb_b};
   // bytes of an operand's K step in its rows
@@ -239,81 +294,92 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
     constexpr int blk = op == 0 ? BLKA : BLKB;
     uint8_t *dst = lds + slot * SB + (blk * wave + j) * 1024;
     const bool lk = KTAIL && c.k == KS - 1;  // (c.k >= 1 there)
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(c.rs, (lds_void *)dst, 16, lk ? vl[op][j & 1] : vo[op][j & 1],
-                                             uint32_t(c.k) * kstep_b[op] + uint32_t(j & ~1) * ld8[op] -
+    constexpr int var = BKN && op == 1 ? kn_var(j) : j & 1;
+    constexpr int past = BKN && op == 1 ? j - kn_rep(j) : j & ~1;  // blocks past the one of those offsets
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(c.rs, (lds_void *)dst, 16, lk ? vl[op][j & 1] : vo[op][var],
+                                             uint32_t(c.k) * kstep_b[op] + uint32_t(past) * ld8[op] -
                                                  (lk ? 16u : 0u),
                                              0, 0);
   };
 
-  const int frow = lane & 31, fg = lane >> 5;
-  int ro[2][2][2];
+  // Fragment f (A blocks 0 .. FM-1, then B blocks) is 16 rows x 128 bytes of
+  // K: lane l holds row l % 16, 16-byte pieces x = 0, 1 = logical chunks
+  // 4x + l / 16 (16-bit: piece x is K half x, one 16x16x32 MFMA; fp8: both
+  // pieces are one 16x16x128 MFMA; the order of K inside a product is the
+  // same for A and B).  Blocks 16 rows apart share the swizzle.
+  const int frow = lane & 15, fg = lane >> 4;
+  int ro[2][2];
 #pragma unroll
-  for (int h = 0; h < 2; ++h)
-#pragma unroll
-    for (int e = 0; e < 2; ++e) {
-      const int chunk = 4 * h + (C::FP8 ? fg + 2 * e : 2 * fg + e);
-      ro[0][h][e] = off(wm * TM + frow, chunk);
-      ro[1][h][e] = off(wn * TN + frow, chunk);
-    }
-  // BKN: the B fragment reads' lane offsets in a slot, per 32-column block
-  // fn, for K row 16 g + s / 4 (g = lane / 32, s = lane mod 16) and columns
-  // 32 fn + 16 ((lane / 16) mod 2) + 4 (s mod 4) .. + 3 of the wave's; half
-  // h, piece e and read r add K rows 32 h + 8 e + 4 r (a multiple of 4, so
-  // the swizzle is the lane's).
+  for (int x = 0; x < 2; ++x) {
+    ro[0][x] = off(wm * TM + frow, 4 * x + fg);
+    ro[1][x] = off(wn * TN + frow, 4 * x + fg);
+  }
+  // BKN: the B fragment reads' lane offsets in a slot, per 16-column block
+  // fn, for K row 8 g + s / 4 (g = lane / 16, s = lane mod 16) and columns
+  // 16 fn + 4 (s mod 4) .. + 3 of the wave's; half h and read r add K rows
+  // 32 h + 4 r (which leave the swizzle alone).
   int bko[BKN ? FN : 1];
   const uint32_t lds_base = uint32_t(reinterpret_cast<uintptr_t>((lds_u8 *)lds));
   if constexpr (BKN) {
-    const int s16 = lane & 15, rho = s16 >> 2;
+    const int s16 = lane & 15, kr = 8 * fg + (s16 >> 2);
 #pragma unroll
     for (int fn = 0; fn < FN; ++fn) {
-      const int n = wn * TN + 32 * fn + 16 * ((lane >> 4) & 1) + 4 * (s16 & 3);
-      bko[fn] = (16 * fg + rho) * KRB + (((n >> 3) ^ persist::kn_swz(rho, KRB)) << 4) + 8 * ((n >> 2) & 1);
+      const int n = wn * TN + 16 * fn + 4 * (s16 & 3);
+      bko[fn] = kr * KRB + (((n >> 3) ^ persist::kn_swz(kr, KRB)) << 4) + 8 * ((n >> 2) & 1);
     }
   }
-  txd::i32x4 fr[2][NF][2];
-  auto read = [&](int slot_a, int slot_b, auto h_tag, auto r_tag) {
-    constexpr int h = decltype(h_tag)::value, r = decltype(r_tag)::value, e = r % 2, o = r / 2;
-    constexpr int f = o == 0 ? 0 : o == 1 ? FM : o <= FM ? o - 1 : o;
-    const uint8_t *Sp = lds + (f < FM ? slot_a : slot_b) * SB;
+  txd::i32x4 fr[NF][2];
+  // Read piece x of fragment f from the step in slots slot_a, slot_b.
+  auto read_piece = [&](int slot_a, int slot_b, auto f_tag, auto x_tag) {
+    constexpr int f = decltype(f_tag)::value, x = decltype(x_tag)::value;
     if constexpr (BKN && f >= FM) {
       // Inline asm: the compiler puts a vmcnt(0) (a drain of every operand
       // load in flight) before the intrinsic form of this read whenever an
       // LDS-DMA load is pending.  Its results are waited for explicitly:
       // kn_wait in the K step's first half, the barrier in the second.
-      constexpr int c0 = (32 * h + 8 * e) * KRB;
+      constexpr int c0 = 32 * x * KRB;
       const uint32_t addr = lds_base + uint32_t(slot_b * SB + bko[f - FM]);
       txd::u32x2 lo, hi;
       asm volatile("ds_read_b64_tr_b16 %0, %2 offset:%3\n\tds_read_b64_tr_b16 %1, %2 offset:%4"
                    : "=&v"(lo), "=&v"(hi)
                    : "v"(addr), "i"(c0), "i"(c0 + 4 * KRB)
                    : "memory");
-      fr[h][f][e] = txd::i32x4{int(lo[0]), int(lo[1]), int(hi[0]), int(hi[1])};
+      fr[f][x] = txd::i32x4{int(lo[0]), int(lo[1]), int(hi[0]), int(hi[1])};
     } else {
-      const int byte = f < FM ? ro[0][h][e] + 4096 * f : ro[1][h][e] + 4096 * (f - FM);
-      fr[h][f][e] = *reinterpret_cast<const txd::i32x4 *>(Sp + byte);
+      const uint8_t *Sp = lds + (f < FM ? slot_a : slot_b) * SB;
+      const int byte = f < FM ? ro[0][x] + 2048 * f : ro[1][x] + 2048 * (f - FM);
+      fr[f][x] = *reinterpret_cast<const txd::i32x4 *>(Sp + byte);
     }
   };
-  // BKN: wait for the first half's B block fn before its first MFMA.  The
-  // half's reads are issued in the order of `read`: A0 (2 LDS operations),
-  // B0 (4), A1 .. A(FM-1) (2 each), B1 .. B(FN-1) (4 each); LDS operations complete
-  // in order, so at most the operations issued after B fn may be left
-  // outstanding (capped at lgkmcnt's 15; extra scalar loads in flight only
-  // make the wait longer).  The asm ties the fragments to the wait.
+  // Read r of K half h (16-bit), in the order the MFMAs consume them: A0, B0,
+  // A1 .. A(FM-1), B1 .. B(FN-1).
+  auto read = [&](int slot_a, int slot_b, auto h_tag, auto r_tag) {
+    constexpr int o = decltype(r_tag)::value, f = o == 0 ? 0 : o == 1 ? FM : o <= FM ? o - 1 : o;
+    read_piece(slot_a, slot_b, std::integral_constant<int, f>{}, h_tag);
+  };
+  // LDS operations of reads 0 .. r - 1 of a K half (BKN: two per B block).
+  constexpr auto read_ops = [](int r) constexpr { return r + (r >= 2 ? 1 : 0) + (r > FM + 1 ? r - FM - 1 : 0); };
+  // BKN: wait for the first half's B block fn before its first MFMA.  LDS
+  // operations complete in order, so at most the operations issued after B
+  // fn may be left outstanding: the rest of that half's reads and the second
+  // half's issued so far (capped at lgkmcnt's 15; extra scalar loads in
+  // flight only make the wait longer).  The asm ties the fragment to the wait.
   auto kn_wait = [&](auto fn_tag) {
     constexpr int fn = decltype(fn_tag)::value;
-    constexpr int after = fn == 0 ? 2 * (FM - 1) + 4 * (FN - 1) : 4 * (FN - 1 - fn);
+    constexpr int after = read_ops(NR) - read_ops(fn == 0 ? 2 : FM + fn + 1) + read_ops(spread_lo(fn * FM, NR, RW));
     constexpr int n = after > 15 ? 15 : after;
-    persist::lgkm_wait_tie<n>(fr[0][FM + fn][0], fr[0][FM + fn][1]);
+    persist::lgkm_wait_tie<n>(fr[FM + fn][0]);
   };
-  txd::f32x16 acc[FN][FM];
-  // MFMA i of a K half: B block i / FM against A block i % FM; FIRST: the
-  // tile's first step, from a zero accumulator.
-  auto mma = [&](auto h_tag, auto i_tag, auto first_tag) {
-    constexpr int h = decltype(h_tag)::value, i = decltype(i_tag)::value, fn = i / FM, fm = i % FM;
-    const i32x8 va = __builtin_shufflevector(fr[h][fm][0], fr[h][fm][1], 0, 1, 2, 3, 4, 5, 6, 7);
-    const i32x8 vb = __builtin_shufflevector(fr[h][FM + fn][0], fr[h][FM + fn][1], 0, 1, 2, 3, 4, 5, 6, 7);
-    if constexpr (decltype(first_tag)::value && h == 0) acc[fn][fm] = txd::f32x16{};
-    mfma32<C>(acc[fn][fm], vb, va);
+  txd::f32x4 acc[FN][FM];
+  // The MFMA of B block fn against A block fm on K half h (fp8: the whole
+  // step); ZERO: the block's first of the tile, from a zero accumulator.
+  auto mma = [&](auto h_tag, auto fn_tag, auto fm_tag, auto zero_tag) {
+    constexpr int h = decltype(h_tag)::value, fn = decltype(fn_tag)::value, fm = decltype(fm_tag)::value;
+    if constexpr (decltype(zero_tag)::value) acc[fn][fm] = txd::f32x4{};
+    persist::mfma16<C>(acc[fn][fm], fr[FM + fn], fr[fm], h);
+    // (kept in its AGPRs: left alone the ragged-K variant rotates blocks
+    // through VGPRs and spills 26 of them)
+    if constexpr (KTAIL) asm volatile("" : "+a"(acc[fn][fm]));
   };
   using H0 = std::integral_constant<int, 0>;
   using H1 = std::integral_constant<int, 1>;
@@ -334,10 +400,28 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
   static_for<BLKA>([&](auto j) { load_op(ca, 4, OpA{}, j); });
   advance(ca, OpA{});  // next A load: step 3
   wait_and_barrier<2 * BLKA + BLKB>();
-  static_for<NR>([&](auto r) { read(0, 1, H0{}, r); });
+  // The fragments a step starts with: 16-bit, its first K half; fp8, all of A
+  // and the first two B blocks.
+  auto read_start = [&](int slot_a, int slot_b) {
+    if constexpr (C::FP8) {
+      static_for<FM + 2>([&](auto f) {
+        read_piece(slot_a, slot_b, f, H0{});
+        read_piece(slot_a, slot_b, f, H1{});
+      });
+    } else {
+      static_for<NR>([&](auto r) { read(slot_a, slot_b, H0{}, r); });
+    }
+  };
+  read_start(0, 1);
 
-  // One K step: half 0 (reads of half 1), barrier, half 1 (loads of B s+2
-  // and A s+3, reads of half 0 of step s+1).  FIRST: the tile's first step
+  // One K step: half 0 (reads of the rest of the step's fragments), barrier,
+  // half 1 (loads of B s+2 and A s+3, reads of the first fragments of step
+  // s+1).  16-bit: half h is K half h of all blocks.  fp8, whose MFMA takes
+  // the whole step's K: half 0 is B blocks 0 .. FN/2-1, block by block, half 1
+  // the others, A block by A block: each A block's registers are reloaded
+  // with step s+1 right after its last MFMA, so fragments take 112 registers
+  // (A 64, four B blocks in use and two ahead).
+  // FIRST: the tile's first step
   // (MFMAs from a zero accumulator); VM: loads and stores allowed in flight
   // at the barrier (the next step's operands are older than the last VM);
   // LAST: the tile's last step, whose A s+3 loads wait until after the
@@ -349,36 +433,67 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
     constexpr bool LAST = decltype(last_tag)::value;
     const int na = sa >= 3 ? sa - 3 : sa + 2, nb = sb >= 3 ? sb - 3 : sb + 2;
     const bool clear = KTAIL && LAST && kt.cp < 8;
-    if (clear) ktail_clear<NF>(fr[0], 0, fg, kt);
+    if (clear) persist::ktail_clear<NF>(fr, 0, fg, kt);
     static_for<NM>([&](auto I) {
       constexpr int i = decltype(I)::value;
-      if constexpr (BKN && i % FM == 0) kn_wait(std::integral_constant<int, i / FM>{});
-      mma(H0{}, I, first_tag);
+      using Fn = std::integral_constant<int, i / FM>;
+      using Fm = std::integral_constant<int, i % FM>;
+      if constexpr (BKN && i % FM == 0) kn_wait(Fn{});
+      mma(H0{}, Fn{}, Fm{}, first_tag);
       __builtin_amdgcn_sched_barrier(0);
-      constexpr int r0 = spread_lo(i, NR, RW), r1 = spread_hi(i, NR, RW);
-      static_for<r1 - r0>([&](auto R) { read(sa, sb, H1{}, std::integral_constant<int, r0 + decltype(R)::value>{}); });
+      if constexpr (C::FP8) {
+        // B blocks 2 .. FN-1, two pieces each
+        constexpr int n = 2 * (FN - 2), r0 = spread_lo(i, n, 2 * n), r1 = spread_hi(i, n, 2 * n);
+        static_for<r1 - r0>([&](auto R) {
+          constexpr int r = r0 + decltype(R)::value;
+          read_piece(sa, sb, std::integral_constant<int, FM + 2 + r / 2>{}, std::integral_constant<int, r % 2>{});
+        });
+      } else {
+        constexpr int r0 = spread_lo(i, NR, RW), r1 = spread_hi(i, NR, RW);
+        static_for<r1 - r0>(
+            [&](auto R) { read(sa, sb, H1{}, std::integral_constant<int, r0 + decltype(R)::value>{}); });
+      }
       __builtin_amdgcn_sched_barrier(0);
     });
     wait_and_barrier<VM>();
     if constexpr (BKN) {
       // the barrier's lgkmcnt(0) completed the second half's B reads
-      static_for<FN>([&](auto fn) { persist::tie(fr[1][FM + decltype(fn)::value][0], fr[1][FM + decltype(fn)::value][1]); });
+      static_for<FN>([&](auto fn) { persist::tie(fr[FM + decltype(fn)::value][1]); });
     }
     __builtin_amdgcn_sched_barrier(0);
-    if (clear) ktail_clear<NF>(fr[1], 1, fg, kt);
+    if (clear) persist::ktail_clear<NF>(fr, 1, fg, kt);
     static_for<NM>([&](auto I) {
       constexpr int i = decltype(I)::value;
-      mma(H1{}, I, std::false_type{});
+      constexpr int HF = FN / 2;
+      if constexpr (C::FP8)
+        mma(H1{}, std::integral_constant<int, HF + i % HF>{}, std::integral_constant<int, i / HF>{}, first_tag);
+      else
+        mma(H1{}, std::integral_constant<int, i / FM>{}, std::integral_constant<int, i % FM>{}, std::false_type{});
       __builtin_amdgcn_sched_barrier(0);
-      constexpr int d0 = spread_lo(i, ND, NM), d1 = spread_hi(i, ND, NM);
+      // operand loads half a run of MFMAs away from the (16-bit) fragment reads
+      constexpr auto nd = [](int j) constexpr {
+        return j <= 0 ? 0 : j >= NM ? ND : (j + (C::FP8 ? 0 : NM / ND / 2)) * ND / NM;
+      };
+      constexpr int d0 = nd(i), d1 = nd(i + 1);
       static_for<d1 - d0>([&](auto D) {
         constexpr int d = d0 + decltype(D)::value;
         if constexpr (d < BLKB) load_op(cb, sa, OpB{}, std::integral_constant<int, d>{});
         else if constexpr (!LAST) load_op(ca, sb, OpA{}, std::integral_constant<int, d - BLKB>{});
       });
-      constexpr int r0 = spread_lo(i, NR, RW), r1 = spread_hi(i, NR, RW);
-      if constexpr (!LAST)
-        static_for<r1 - r0>([&](auto R) { read(na, nb, H0{}, std::integral_constant<int, r0 + decltype(R)::value>{}); });
+      if constexpr (!LAST && C::FP8) {
+        // A block i / HF after its last MFMA (the second piece one MFMA on),
+        // B blocks 0 and 1 in between
+        constexpr int g = i / HF, j = i % HF;
+        if constexpr (j == HF - 1) read_piece(na, nb, std::integral_constant<int, g>{}, H0{});
+        if constexpr (j == 0 && g > 0) read_piece(na, nb, std::integral_constant<int, g - 1>{}, H1{});
+        if constexpr (j == 1 && g < 4)
+          read_piece(na, nb, std::integral_constant<int, FM + g / 2>{}, std::integral_constant<int, g % 2>{});
+        if constexpr (i == NM - 1) read_piece(na, nb, std::integral_constant<int, FM - 1>{}, H1{});
+      } else if constexpr (!LAST) {
+        constexpr int r0 = spread_lo(i, NR, NM), r1 = spread_hi(i, NR, NM);
+        static_for<r1 - r0>(
+            [&](auto R) { read(na, nb, H0{}, std::integral_constant<int, r0 + decltype(R)::value>{}); });
+      }
       __builtin_amdgcn_sched_barrier(0);
     });
     advance(cb, OpB{});
@@ -393,12 +508,12 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
   // staging geometry: the wave's 32 x TN block as 32 rows of SRB bytes
   // (CH 16-byte chunks), read back SPI rows per instruction
   constexpr int SRB = 2 * TN, CH = SRB / 16, SPI = 64 / CH;
-  constexpr int kEpiStores = FM * (32 / SPI);
+  constexpr int kEpiStores = FM / 2 * (32 / SPI);
   using VmAfterEpi = std::integral_constant<int, BLKB + kEpiStores>;
   static_assert(BLKB + kEpiStores < 64, "vmcnt range");
-  // Scale loads issued before the last step (row scales, 16 column-scale
+  // Scale loads issued before the last step (row scales, column-scale
   // vectors) that its barrier leaves in flight with the step's own A loads.
-  constexpr int kScaleLoads = ROWCOL ? FM + 4 * FN : 0;
+  constexpr int kScaleLoads = ROWCOL ? FM + FN : 0;
   using VmLast = std::integral_constant<int, BLKA + kScaleLoads>;
   static_assert(BLKA + kScaleLoads < 64, "vmcnt range");
 
@@ -428,21 +543,19 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
     // load).  Rows past M read row M - 1 and columns past N the last four;
     // their stores are dropped.
     float sav[FM];
-    txd::f32x4 sb4[FN][4];  // columns 32 fn + 8 jj + 4 g .. + 3 of the wave's
+    txd::f32x4 sb4[FN];  // columns 16 fn + 4 g .. + 3 of the wave's
     if constexpr (ROWCOL) {
       const int nl = n0 + wn * TN + 4 * fg;
 #pragma unroll
       for (int fm = 0; fm < FM; ++fm) {
-        const float *ps = d.sa + min(m0 + wm * TM + fm * 32 + frow, d.rows - 1);
+        const float *ps = d.sa + min(m0 + wm * TM + fm * 16 + frow, d.rows - 1);
         asm volatile("global_load_dword %0, %1, off" : "=v"(sav[fm]) : "v"(ps) : "memory");
       }
 #pragma unroll
-      for (int fn = 0; fn < FN; ++fn)
-#pragma unroll
-        for (int jj = 0; jj < 4; ++jj) {
-          const float *ps = d.sb + min(nl + 32 * fn + 8 * jj, a.N - 4);
-          asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(sb4[fn][jj]) : "v"(ps) : "memory");
-        }
+      for (int fn = 0; fn < FN; ++fn) {
+        const float *ps = d.sb + min(nl + 16 * fn, a.N - 4);
+        asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(sb4[fn]) : "v"(ps) : "memory");
+      }
     }
     const int stage_slot = sb;  // the last step's B slot: its A s+3 loads go there
     step(std::false_type{}, VmLast{}, std::true_type{});  // the last step (KS >= 2)
@@ -451,17 +564,15 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
 #pragma unroll
       for (int fm = 0; fm < FM; ++fm) asm volatile("" : "+v"(sav[fm]));
 #pragma unroll
-      for (int fn = 0; fn < FN; ++fn)
-        asm volatile("" : "+v"(sb4[fn][0]), "+v"(sb4[fn][1]), "+v"(sb4[fn][2]), "+v"(sb4[fn][3]));
+      for (int fn = 0; fn < FN; ++fn) asm volatile("" : "+v"(sb4[fn]));
     }
-    // Epilogue, per 32-row block fm: scale, round, and exchange halves so
-    // that lane l < 32 holds columns 16 p .. 16 p + 7 and lane l + 32
-    // columns 16 p + 8 .. + 15 of row l % 32 (p = 2 fn + pr); stage the
-    // wave's 32 x TN block, then store SPI rows of SRB bytes per instruction.
+    // Epilogue, per 32-row block: scale, round and stage the wave's 32 x TN
+    // block (lane l: 4 columns 16 fn + 4 (l / 16) .. of row l % 16 of each 16 x
+    // 16 block), then store SPI rows of SRB bytes per instruction.
     // The accumulators are read below in inline asm, for which the compiler
     // inserts no wait states after the MFMAs that write them: the last step's
-    // final MFMAs stay above this point, and 32 wait states (a 16-pass MFMA's
-    // result needs about 19) pass before the first read.
+    // final MFMAs stay above this point, and 32 wait states (an 8-pass MFMA's
+    // result needs about 11) pass before the first read.
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
@@ -471,47 +582,35 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
     // registers through the whole K loop (fp8: 238 -> 206 VGPRs).
     int el = lane;
     asm volatile("" : "+v"(el));
-    const int efrow = el & 31, efg = el >> 5;
+    const int efrow = el & 15, efg = el >> 4;
     const int srow = el / CH, schunk = el % CH;  // read-back: row SPI i + srow, chunk schunk
     const int n_st = n0 + wn * TN + 8 * schunk;
     const uint32_t coloff = n_st < a.N ? uint32_t(n_st) * 2u + cmis : kOob;
-    static_for<FM>([&](auto fm_tag) {
-      constexpr int fm = decltype(fm_tag)::value;
-      static_for<FN>([&](auto fn_tag) {
-        constexpr int fn = decltype(fn_tag)::value;
+    static_for<FM / 2>([&](auto blk_tag) {
+      constexpr int blk = decltype(blk_tag)::value;
+      static_for<2>([&](auto u_tag) {
+        constexpr int u = decltype(u_tag)::value, fm = 2 * blk + u;
+        static_for<FN>([&](auto fn_tag) {
+          constexpr int fn = decltype(fn_tag)::value;
+          float v[4];
 #pragma unroll
-        for (int pr = 0; pr < 2; ++pr) {
-          uint32_t pk[2][2];
-#pragma unroll
-          for (int jl = 0; jl < 2; ++jl) {
-            float v[4];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              // read the accumulator where it is used (the compiler would
-              // otherwise copy whole tiles out of the AGPRs at once)
-              asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(v[q]) : "a"(acc[fn][fm][4 * (2 * pr + jl) + q]));
-              if constexpr (ROWCOL) v[q] = v[q] * sav[fm] * sb4[fn][2 * pr + jl][q];
-            }
-            pk[jl][0] = OUT == OUT_F16 ? txd::pack_f16x2(v[0], v[1]) : txd::pack_bf16x2(v[0], v[1]);
-            pk[jl][1] = OUT == OUT_F16 ? txd::pack_f16x2(v[2], v[3]) : txd::pack_bf16x2(v[2], v[3]);
+          for (int q = 0; q < 4; ++q) {
+            // read the accumulator where it is used (the compiler would
+            // otherwise copy whole tiles out of the AGPRs at once)
+            asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(v[q]) : "a"(acc[fn][fm][q]));
+            if constexpr (ROWCOL) v[q] = v[q] * sav[fm] * sb4[fn][q];
           }
-          uint32_t o[4];
-#pragma unroll
-          for (int d = 0; d < 2; ++d) {
-            const auto sw = __builtin_amdgcn_permlane32_swap(pk[0][d], pk[1][d], false, false);
-            o[d] = sw[0];
-            o[2 + d] = sw[1];
-          }
-          const int chunk = 2 * (2 * fn + pr) + efg;
-          *reinterpret_cast<txd::u32x4 *>(stg + efrow * SRB + ((chunk ^ (efrow & (CH - 1))) << 4)) =
-              txd::u32x4{o[0], o[1], o[2], o[3]};
-        }
+          const int row = 16 * u + efrow, chunk = 2 * fn + (efg >> 1);
+          *reinterpret_cast<txd::u32x2 *>(stg + row * SRB + ((chunk ^ (row & (CH - 1))) << 4) + 8 * (efg & 1)) =
+              OUT == OUT_F16 ? txd::u32x2{txd::pack_f16x2(v[0], v[1]), txd::pack_f16x2(v[2], v[3])}
+                             : txd::u32x2{txd::pack_bf16x2(v[0], v[1]), txd::pack_bf16x2(v[2], v[3])};
+        });
       });
 #pragma unroll
       for (int i = 0; i < 32 / SPI; ++i) {
         const int r = SPI * i + srow;
         const txd::u32x4 w = *reinterpret_cast<const txd::u32x4 *>(stg + r * SRB + ((schunk ^ (r & (CH - 1))) << 4));
-        const int m = m0 + wm * TM + fm * 32 + r;
+        const int m = m0 + wm * TM + blk * 32 + r;
         const uint32_t voff = (m >= d.rows || coloff == kOob) ? kOob : uint32_t(m) * uint32_t(a.ldc) * 2u + coloff;
         __builtin_amdgcn_raw_buffer_store_b128(w, crs, voff, 0, 0);
       }
@@ -521,7 +620,7 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
     __builtin_amdgcn_s_waitcnt((63 & 15) | (7 << 4) | (0 << 8) | ((63 >> 4) << 14));
     static_for<BLKA>([&](auto j) { load_op(ca, stage_slot, OpA{}, j); });
     advance(ca, OpA{});
-    static_for<NR>([&](auto r) { read(sa, sb, H0{}, r); });
+    read_start(sa, sb);
   }
   // Drain the trailing (empty-range) loads before the workgroup's LDS is released.
   wait_and_barrier<0>();
