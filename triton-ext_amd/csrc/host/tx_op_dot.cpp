@@ -418,6 +418,50 @@ static int persist_kn_tile(const tx_gemm_args &args) {
   return ok ? bt : 0;
 }
 
+// tt.dot with 16-bit operands and an fp32 output D = A.B + C in one launch of
+// the persistent tile (gemm_persist.h, OUT_F32), where dot16 would take that
+// tile too: a 256-, 128- or 64-wide tile by the same rule, K a whole number
+// (>= 2) of 64-element steps (ragged K: the 256-wide tile, N x K B only), N a
+// multiple of 4, C and D and their rows 16-byte aligned, every matrix
+// addressable with 32-bit byte offsets.  TX_UNSUPPORTED (nothing launched)
+// otherwise: too few tiles with a long K want the K split's planes.
+static tx_status launch_acc_persist(const char *pfx, tx_gemm_args args, bool kn, hipStream_t s) {
+  const int64_t M = args.M, N = args.N, K = args.K, cus = cu_count(), lim = int64_t(1) << 31;
+  const int64_t kb = K * 2;
+  if (N % 4 || kb < 256 || !aligned(args.C, 16) || args.ldc % 4 || (M - 1) * args.ldc * 4 + N * 4 >= lim ||
+      (args.acc && (!aligned(args.acc, 16) || args.ld_acc % 4 || (M - 1) * args.ld_acc * 4 + N * 4 >= lim)))
+    return TX_UNSUPPORTED;
+  const bool whole = kb % 128 == 0;
+  int bt = 256;
+  if (((M + 255) / 256) * ((N + 255) / 256) < cus) bt = small_persist_tile(M, N, kb, cus);
+  if (!bt || (!whole && (kn || bt != 256))) return TX_UNSUPPORTED;
+  if (kn) {
+    if (!aligned(args.A, 16) || args.lda % 8 || !aligned(args.B, 16) || args.ldb % 8 || N % 8 ||
+        (M - 1) * args.lda * 2 + kb + 16 >= lim || (K - 1) * args.ldb * 2 + N * 2 + 512 >= lim)
+      return TX_UNSUPPORTED;
+  } else if (whole ? !fast_ok(args.A, args.lda * 2, args.B, args.ldb * 2, kb, M, N)
+                   : !fast16_ragged_ok(args.A, args.lda * 2, args.B, args.ldb * 2, kb, M, N)) {
+    return TX_UNSUPPORTED;
+  }
+  char kname[96], tile[8] = "";
+  if (bt != 256) {
+    std::snprintf(tile, sizeof tile, "%d", bt);
+    // K segments: as many as launch_acc would split K into, so that the sums
+    // round no worse
+    const int64_t tiles = ((M + 255) / 256) * ((N + 127) / 128), ksteps = kb / 128;
+    const int64_t splits = std::max<int64_t>(1, std::min({kMaxSplits, cus / tiles, ksteps / kMinStepsPerSplit}));
+    args.ksteps_split = splits > 1 ? int32_t((ksteps + splits - 1) / splits) : 0;
+  }
+  std::snprintf(kname, sizeof kname, "tx_gemm_%s_fast_acc_persist%s%s", pfx, tile, kn ? "_kn" : whole ? "" : "_kt");
+  args.tiles_m = int32_t((M + bt - 1) / bt);
+  args.tiles_n = int32_t((N + bt - 1) / bt);
+  args.group_m = std::min<int32_t>(kGroupM, args.tiles_m);
+  hipFunction_t fn;
+  TX_TRY(get_kernel(CodeObject::GemmBf16, kname, &fn));
+  const int64_t grid = std::min<int64_t>(int64_t(args.tiles_m) * args.tiles_n, cus);
+  return launch(fn, unsigned(grid), 1, 64 * kPersistWaves, s, &args, sizeof args, kname);
+}
+
 // tt.dot with 16-bit operands (bf16 / fp16) and a 16-bit output.  Kernel
 // names: tx_gemm_<operands>_<variant>[_out_<output>]; the split-K reduce
 // is the output type's.
@@ -662,6 +706,12 @@ static tx_status dot_acc(const void *A, tx_dtype a_type, int64_t lda, const floa
   else std::snprintf(base, sizeof base, "tx_gemm_%s_fast", a_type == TX_BF16 ? "bf16" : "f16");
   const char *reduce = fp8 ? "tx_gemm_fp8_splitk_reduce" : "tx_gemm_bf16_splitk_reduce";
   if (K == 0) return launch_acc(base, reduce, co, args, 0, s);
+  if (b16 && d_type == TX_F32) {
+    // one launch of the persistent tile (nothing launched: TX_UNSUPPORTED)
+    const tx_status st = launch_acc_persist(a_type == TX_BF16 ? "bf16" : "f16", args, kn, s);
+    if (st != TX_UNSUPPORTED) return st;
+    clear_error();
+  }
   ScratchLease ws;  // operand copies (slot 0), held until the product is enqueued
   if (kn) {
     TX_TRY(transpose_kn(what, args, s, ws));

@@ -92,6 +92,15 @@ TX_GEMM16_PERSIST(bf16, EL_BF16, _out_f16, OUT_F16)
 TX_GEMM16_PERSIST(f16, EL_F16, , OUT_F16)
 TX_GEMM16_PERSIST(f16, EL_F16, _out_bf16, OUT_BF16)
 
+// tt.dot with its accumulator operand, D = A.B + C in fp32 (a.acc, NULL: no
+// C), on the persistent tiles: tx_gemm_{bf16,f16}_fast_acc_persist...  The
+// 256 x 128 tile's fp32 planes and the reduce that adds C moved 8 M N bytes
+// per split and cost a launch (and a row-major B a transpose).  Before ->
+// here, same box: bf16 2048^3 49 -> 27 us, 4096^3 187 -> 114 us, 4096 x 4096 x
+// 128 row-major B 83 -> 28 us, 640 x 2000 x 3968 row-major B 38 -> 35 us.
+TX_GEMM16_PERSIST(bf16, EL_BF16, _acc, OUT_F32)
+TX_GEMM16_PERSIST(f16, EL_F16, _acc, OUT_F32)
+
 // Column strip of a 16-bit product: C[:, 0 .. N) with N <= W (1, 2, 4 or
 // 8), the few columns past the last 256-column block of a larger product
 // (whose 256-row tiles would spend a whole tile of MFMAs on each).  VALU dot

@@ -28,7 +28,8 @@
 // accumulators in place, moves nothing beyond 1%).
 //
 // The K loop is that of gemm_fast_tile_at (ring of 5 LDS slots of BT x 128 bytes,
-// B of step s+2 and A of step s+3 loaded during the second half of step s,
+// B of step s+2 and A of step s+3 loaded during the second half of step s; BT
+// below 256: 5 or 8 stages of a whole step, both of step s+5 or s+8,
 // fragments one 64-byte half ahead in registers, one barrier per step), with
 // s counting steps over all tiles of the workgroup.  Each operand's loads go
 // through a buffer resource for the tile they belong to: base at the tile's
@@ -50,7 +51,10 @@
 // wave writes its 32 x BT / 2 block to its own quarter of that slot, reads
 // back whole rows (BT = 256: 4 of 256 bytes) per instruction and stores them
 // through a buffer
-// resource for C (stores past M / N are dropped).  The first K step of each
+// resource for C (stores past M / N are dropped).  OUT_F32 (tt.dot with its
+// accumulator operand): D = A.B + C in fp32 is written straight from the
+// accumulators, C's loads for the first row blocks issued before the last K
+// step.  The first K step of each
 // tile starts its MFMAs from a zero accumulator operand, so the accumulators
 // are never cleared explicitly.
 #pragma once
@@ -142,7 +146,9 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rsrc(const void *base, in
 template <class C, int OUT = OUT_BF16, bool GROUPED = false, bool KTAIL = false, bool BKN = false, int BT = 256>
 __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_grouped_args *q = nullptr) {
   using namespace fast;
-  static_assert(OUT == OUT_BF16 || (OUT == OUT_F16 && !C::FP8), "bf16 output, or fp16 out of 16-bit operands");
+  static_assert(OUT == OUT_BF16 || (OUT == OUT_F16 && !C::FP8) || (OUT == OUT_F32 && !C::FP8),
+                "bf16 output, or fp16 / fp32 (+ accumulator) out of 16-bit operands");
+  constexpr bool F32 = OUT == OUT_F32;
   static_assert(!KTAIL || (!C::FP8 && !GROUPED), "ragged K: 16-bit operands, one product");
   static_assert(!BKN || (!C::FP8 && !GROUPED && !KTAIL), "row-major B: 16-bit operands, whole K steps");
   static_assert(BT == 256 || BT == 128 || BT == 64, "tile 256, 128 or 64 square");
@@ -154,10 +160,17 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
   constexpr int SB = BT * kStep;  // one operand of one K step
   constexpr int BLKA = SB / 1024 / NW, BLKB = BLKA, ND = BLKA + BLKB;
   constexpr int RW = NM >= 2 ? NM / 2 : 1;
+  // Ring: BT = 256, 5 slots of one operand of one step (B two steps ahead, A
+  // three); smaller tiles, whose step is a fraction of the time a load
+  // takes to arrive, D stages of a step's A and B slots, both loaded D steps
+  // ahead (160 and 128 KiB): against the 5-slot ring fp16 640 x 2000 x 3968
+  // (BT = 64) 51.7 -> 33.0 us, 2304 x 2304 x 4096 (BT = 128) 68.1 -> 59.7.
+  constexpr bool STG = BT < 256;
+  constexpr int D = BT == 128 ? 5 : 8, NSLOT = STG ? 2 * D : kSlots;
   constexpr bool ROWCOL = C::FP8;
   // BKN: bytes of a K row of the B tile, and K rows per 1 KiB DMA block
   constexpr int KRB = 2 * BT, RPB = 1024 / KRB, CPR = KRB / 16;
-  __shared__ __attribute__((aligned(1024))) uint8_t lds[kSlots * SB];
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[NSLOT * SB];
 
   // m tiles: the grouped product's real count is only on the device
   const int tiles_m = GROUPED ? q->tile_prefix[q->groups] : a.tiles_m;
@@ -378,28 +391,33 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
     if constexpr (decltype(zero_tag)::value) acc[fn][fm] = txd::f32x4{};
     persist::mfma16<C>(acc[fn][fm], fr[FM + fn], fr[fm], h);
     // (kept in its AGPRs: left alone the ragged-K variant rotates blocks
-    // through VGPRs and spills 26 of them)
-    if constexpr (KTAIL) asm volatile("" : "+a"(acc[fn][fm]));
+    // through VGPRs and spills 26 of them, and the fp32 one copies them)
+    if constexpr (KTAIL || (F32 && BT < 256)) asm volatile("" : "+a"(acc[fn][fm]));
   };
   using H0 = std::integral_constant<int, 0>;
   using H1 = std::integral_constant<int, 1>;
 
-  // Prologue: steps 0, 0, 1, 1, 2 (A0 B0 A1 B1 A2) of the first tile.
+  // Prologue: steps 0, 0, 1, 1, 2 (A0 B0 A1 B1 A2) of the first tile (STG:
+  // A and B of its first D steps).
   Cursor ca, cb;
   ca.t = ca.k = cb.t = cb.k = 0;
   set_tile(ca, OpA{});
   set_tile(cb, OpB{});
-  static_for<BLKA>([&](auto j) { load_op(ca, 0, OpA{}, j); });
-  static_for<BLKB>([&](auto j) { load_op(cb, 1, OpB{}, j); });
-  advance(ca, OpA{});
-  advance(cb, OpB{});
-  static_for<BLKA>([&](auto j) { load_op(ca, 2, OpA{}, j); });
-  static_for<BLKB>([&](auto j) { load_op(cb, 3, OpB{}, j); });
-  advance(ca, OpA{});
-  advance(cb, OpB{});  // next B load: step 2
-  static_for<BLKA>([&](auto j) { load_op(ca, 4, OpA{}, j); });
-  advance(ca, OpA{});  // next A load: step 3
-  wait_and_barrier<2 * BLKA + BLKB>();
+  static_for<STG ? D : 2>([&](auto st) {
+    constexpr int sl = 2 * decltype(st)::value;
+    static_for<BLKA>([&](auto j) { load_op(ca, sl, OpA{}, j); });
+    static_for<BLKB>([&](auto j) { load_op(cb, sl + 1, OpB{}, j); });
+    advance(ca, OpA{});
+    advance(cb, OpB{});
+  });
+  if constexpr (STG) {
+    wait_and_barrier<(D - 1) * ND>();
+  } else {
+    // (next B load: step 2, next A load: step 3)
+    static_for<BLKA>([&](auto j) { load_op(ca, 4, OpA{}, j); });
+    advance(ca, OpA{});
+    wait_and_barrier<2 * BLKA + BLKB>();
+  }
   // The fragments a step starts with: 16-bit, its first K half; fp8, all of A
   // and the first two B blocks.
   auto read_start = [&](int slot_a, int slot_b) {
@@ -431,7 +449,10 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
   auto step = [&](auto first_tag, auto vm_tag, auto last_tag) {
     constexpr int VM = decltype(vm_tag)::value;
     constexpr bool LAST = decltype(last_tag)::value;
-    const int na = sa >= 3 ? sa - 3 : sa + 2, nb = sb >= 3 ? sb - 3 : sb + 2;
+    // slots of step s+1, and those the loads go into (free after the barrier)
+    const int na = STG ? (sa == 2 * (D - 1) ? 0 : sa + 2) : sa >= 3 ? sa - 3 : sa + 2;
+    const int nb = STG ? na + 1 : sb >= 3 ? sb - 3 : sb + 2;
+    const int la = STG ? sa : sb, lb = STG ? sb : sa;
     const bool clear = KTAIL && LAST && kt.cp < 8;
     if (clear) persist::ktail_clear<NF>(fr, 0, fg, kt);
     static_for<NM>([&](auto I) {
@@ -477,8 +498,8 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
       constexpr int d0 = nd(i), d1 = nd(i + 1);
       static_for<d1 - d0>([&](auto D) {
         constexpr int d = d0 + decltype(D)::value;
-        if constexpr (d < BLKB) load_op(cb, sa, OpB{}, std::integral_constant<int, d>{});
-        else if constexpr (!LAST) load_op(ca, sb, OpA{}, std::integral_constant<int, d - BLKB>{});
+        if constexpr (d < BLKB) load_op(cb, lb, OpB{}, std::integral_constant<int, d>{});
+        else if constexpr (!LAST) load_op(ca, la, OpA{}, std::integral_constant<int, d - BLKB>{});
       });
       if constexpr (!LAST && C::FP8) {
         // A block i / HF after its last MFMA (the second piece one MFMA on),
@@ -501,26 +522,39 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
     sa = na;
     sb = nb;
   };
-  using VmStep = std::integral_constant<int, BLKA>;
+  // operand loads the barrier of a step leaves in flight: those of the steps
+  // past s+1
+  constexpr int kAhead = STG ? (D - 2) * ND : BLKA;
+  using VmStep = std::integral_constant<int, kAhead>;
   // The epilogue issues exactly kEpiStores stores per wave, then the last
   // step's deferred BLKA loads of A; the next tile's first barrier may
   // leave all of them in flight.
   // staging geometry: the wave's 32 x TN block as 32 rows of SRB bytes
   // (CH 16-byte chunks), read back SPI rows per instruction
   constexpr int SRB = 2 * TN, CH = SRB / 16, SPI = 64 / CH;
-  constexpr int kEpiStores = FM / 2 * (32 / SPI);
-  using VmAfterEpi = std::integral_constant<int, BLKB + kEpiStores>;
-  static_assert(BLKB + kEpiStores < 64, "vmcnt range");
+  constexpr int kEpiStores = F32 ? FM * FN : FM / 2 * (32 / SPI);
+  constexpr int kAfterEpi = kAhead + kEpiStores + (STG ? 0 : BLKB - BLKA);
+  using VmAfterEpi = std::integral_constant<int, (kAfterEpi < 64 ? kAfterEpi : 63)>;
   // Scale loads issued before the last step (row scales, column-scale
   // vectors) that its barrier leaves in flight with the step's own A loads.
-  constexpr int kScaleLoads = ROWCOL ? FM + FN : 0;
-  using VmLast = std::integral_constant<int, BLKA + kScaleLoads>;
-  static_assert(BLKA + kScaleLoads < 64, "vmcnt range");
+  // F32: the tile's accumulator operand (C), 4 columns per load, is read in
+  // batches of FB row blocks, 16 loads (BT = 64: 4; KTAIL, short of registers:
+  // 8) each, the first before the last step.
+  constexpr int FB = FM < 4 ? FM : KTAIL ? 1 : 16 / FN, NB = FM / FB;
+  constexpr int kScaleLoads = ROWCOL ? FM + FN : F32 ? FB * FN : 0;
+  using VmLast = std::integral_constant<int, kAhead + kScaleLoads>;
+  static_assert(kAhead + kScaleLoads < 64, "vmcnt range");
 
   // Staging: wave w owns bytes 32 SRB w .. + 32 SRB of the slot its last
   // step's A s+3 loads would have filled (the same bytes those loads fill
   // once the epilogue is done, so no other wave ever touches them): 32 rows
   // of SRB bytes, 16-byte chunk c of row r at c ^ (r % CH).
+  // F32 tiles below 256: K in segments of a.ksteps_split steps (0: one),
+  // summed in fp32 registers in order, the rounding of a K split's planes (a
+  // segment's MFMA chain is that much shorter).
+  constexpr bool FOLD = F32 && BT < 256;
+  txd::f32x4 sum[FOLD ? FN : 1][FOLD ? FM : 1];
+  bool folded = false;
   for (int t = 0; t < T; ++t) {
     const TileDesc d = desc(t);
     const int m0 = d.tm * BT, n0 = d.tn * BT;
@@ -530,10 +564,37 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
     // any alignment; the buffer starts at the 16-byte boundary below C.
     const uint32_t cmis = KTAIL ? uint32_t(reinterpret_cast<uintptr_t>(d.out) & 15u) : 0u;
     const __amdgpu_buffer_rsrc_t crs =
-        make_rsrc(d.out - cmis, uint32_t((int64_t(d.rows - 1) * a.ldc + a.N) * 2) + cmis);
+        make_rsrc(d.out - cmis, uint32_t((int64_t(d.rows - 1) * a.ldc + a.N) * (F32 ? 4 : 2)) + cmis);
     if (t == 0) step(std::true_type{}, VmStep{}, std::false_type{});
     else step(std::true_type{}, VmAfterEpi{}, std::false_type{});
-    for (int k = 1; k < KS - 1; ++k) step(std::false_type{}, VmStep{}, std::false_type{});
+    if constexpr (FOLD) {
+      // K segments: at each boundary the accumulators are added to `sum`
+      // and start again from zero
+      const int per = a.ksteps_split > 0 ? a.ksteps_split : KS;
+      folded = KS - per >= 2;
+      if (folded) {
+#pragma unroll
+        for (int fn = 0; fn < FN; ++fn)
+#pragma unroll
+          for (int fm = 0; fm < FM; ++fm) sum[fn][fm] = txd::f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+      // steps between the tile's first and last; none may end on a boundary
+      // just before the last
+      for (int rem = KS - 2, n = min(per - 1, rem);;) {
+        for (int i = 0; i < n; ++i) step(std::false_type{}, VmStep{}, std::false_type{});
+        rem -= n;
+        if (rem == 0) break;
+#pragma unroll
+        for (int fn = 0; fn < FN; ++fn)
+#pragma unroll
+          for (int fm = 0; fm < FM; ++fm) sum[fn][fm] += acc[fn][fm];
+        step(std::true_type{}, VmStep{}, std::false_type{});
+        --rem;
+        n = min(per - 1, rem);
+      }
+    } else {
+      for (int k = 1; k < KS - 1; ++k) step(std::false_type{}, VmStep{}, std::false_type{});
+    }
     // Scales load just before the last step and are waited for after it
     // with vmcnt(BLKB), leaving its B loads in flight.  Loads and waits are
     // written out: the compiler does not count the LDS-DMA loads when it
@@ -557,7 +618,31 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
         asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(sb4[fn]) : "v"(ps) : "memory");
       }
     }
-    const int stage_slot = sb;  // the last step's B slot: its A s+3 loads go there
+    // F32: the accumulator operand through a buffer of its own (empty
+    // without one), element (m, n) of row block fm and column block fn.
+    txd::u32x4 cin[F32 ? 2 : 1][F32 ? FB : 1][F32 ? FN : 1];
+    const __amdgpu_buffer_rsrc_t ars = make_rsrc(
+        a.acc, F32 && a.acc ? uint32_t((int64_t(d.rows - 1) * a.ld_acc + a.N) * 4) : 0u);
+    // byte offset of row block fm, column block fn in a matrix of ld
+    // elements; past M / N, out of any range (N is a multiple of 4 here)
+    auto f32_off = [&](int fm, int fn, int64_t ld) {
+      const int m = m0 + wm * TM + 16 * fm + frow, n = n0 + wn * TN + 16 * fn + 4 * fg;
+      return m < d.rows && n < a.N ? (uint32_t(m) * uint32_t(ld) + uint32_t(n)) * 4u : kOob;
+    };
+    auto load_acc = [&](auto b_tag) {
+      constexpr int b = decltype(b_tag)::value;
+#pragma unroll
+      for (int i = 0; i < FB; ++i)
+#pragma unroll
+        for (int fn = 0; fn < FN; ++fn)
+          cin[b % 2][i][fn] = __builtin_bit_cast(
+              txd::u32x4, __builtin_amdgcn_raw_buffer_load_b128(ars, f32_off(b * FB + i, fn, a.ld_acc), 0, 0));
+    };
+    if constexpr (F32) {
+      load_acc(std::integral_constant<int, 0>{});
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    const int stage_slot = STG ? sa : sb;  // the slot the last step's A loads go to
     step(std::false_type{}, VmLast{}, std::true_type{});  // the last step (KS >= 2)
     if constexpr (ROWCOL) {
       asm volatile("s_waitcnt vmcnt(%0)" ::"n"(BLKB) : "memory");
@@ -576,6 +661,35 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
+    if constexpr (F32) {
+      // D = A.B + C straight from the accumulators: 16 rows of 64 bytes per
+      // store.  Batch b + 1 of C loads ahead of batch b's stores, so its wait
+      // never includes them.
+      static_for<NB>([&](auto b_tag) {
+        constexpr int b = decltype(b_tag)::value;
+        if constexpr (b + 1 < NB) {
+          load_acc(std::integral_constant<int, b + 1>{});
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        static_for<FB>([&](auto i_tag) {
+          constexpr int i = decltype(i_tag)::value, fm = b * FB + i;
+          static_for<FN>([&](auto fn_tag) {
+            constexpr int fn = decltype(fn_tag)::value;
+            txd::u32x4 w;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              float v;
+              asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(v) : "a"(acc[fn][fm][q]));
+              if constexpr (FOLD)
+                if (folded) v = sum[fn][fm][q] + v;
+              w[q] = __float_as_uint(a.acc ? v + __uint_as_float(cin[b % 2][i][fn][q]) : v);
+            }
+            __builtin_amdgcn_raw_buffer_store_b128(w, crs, f32_off(fm, fn, a.ldc), 0, 0);
+          });
+        });
+        __builtin_amdgcn_sched_barrier(0);
+      });
+    }
     uint8_t *stg = lds + stage_slot * SB + wave * (32 * SRB);
     // The lane's staging offsets are recomputed for each tile from an opaque
     // copy of the lane index: hoisted out of the tile loop, they would hold
@@ -586,7 +700,7 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
     const int srow = el / CH, schunk = el % CH;  // read-back: row SPI i + srow, chunk schunk
     const int n_st = n0 + wn * TN + 8 * schunk;
     const uint32_t coloff = n_st < a.N ? uint32_t(n_st) * 2u + cmis : kOob;
-    static_for<FM / 2>([&](auto blk_tag) {
+    if constexpr (!F32) static_for<FM / 2>([&](auto blk_tag) {
       constexpr int blk = decltype(blk_tag)::value;
       static_for<2>([&](auto u_tag) {
         constexpr int u = decltype(u_tag)::value, fm = 2 * blk + u;
