@@ -4,8 +4,9 @@
 // reference.
 //
 // The grouped product needs one workspace: the m-tile prefix sums of its
-// groups (groups + 1 int32), written by a one-workgroup scan before the
-// product reads them.  Here that workspace is a file-scope device array of
+// groups (groups + 1 int32) and, where it fits, the persistent tiles' map (16
+// bytes per m tile), written by a one-workgroup scan before the product reads
+// them.  Here that workspace is a file-scope device array of
 // kNoAllocScratchBytes, one copy per GPU, alive until the process ends.  Its
 // device address is looked up once per device with hipGetSymbolAddress (at
 // txInit, or on the entry point's first call on that device) and only that
@@ -86,7 +87,8 @@ TX_API tx_status tx_dot_fp8_scaled_grouped_noalloc(const void *A, tx_dtype a_typ
   if (groups > 0 && M > 0 && N > 0) TX_TRY(tx::noalloc_scratch(&ws));
   return tx::dot_fp8_scaled_grouped_ws(what, A, a_type, lda, scale_a, B, b_type, ldb, stride_b, scale_b,
                                        stride_scale_b, bias, stride_bias, activation, C, c_type, c_scale, ldc,
-                                       group_offsets, groups, M, N, K, stream, static_cast<int32_t *>(ws));
+                                       group_offsets, groups, M, N, K, stream, static_cast<int32_t *>(ws),
+                                       int64_t(kNoAllocScratchBytes / sizeof(int32_t)));
 }
 
 }  // extern "C"

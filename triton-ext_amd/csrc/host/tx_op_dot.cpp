@@ -930,6 +930,10 @@ static tx_status dot_scaled_mx(const void *A, tx_dtype a_type, int64_t lda, cons
   return launch(fn, unsigned(grid), 1, 256, s, &args, sizeof args, rname);
 }
 
+// Most groups whose tiles are dealt over the XCDs (kOrderMax, gemm_fp8.hip),
+// and most m tiles with a map (1 MiB).
+constexpr int64_t kOrderMaxGroups = 512, kMapMaxTiles = 65536;
+
 // Grouped (offsets != NULL) or batched fp8 scaled dot, bf16 out: the fast
 // tile over every (problem, tile) pair in one launch (tx_grouped_args).  The
 // group sizes stay on the device: a one-workgroup scan turns the offsets
@@ -944,7 +948,8 @@ static tx_status dot_fp8_grouped_impl(const char *what, const void *A, tx_dtype 
                                       int64_t stride_c, const int32_t *offsets, int64_t groups,
                                       int64_t M, int64_t N, int64_t K, tx_stream_t stream,
                                       const Epilogue &e = Epilogue{}, size_t es = 2,
-                                      int64_t stride_bias = 0, int32_t *prefix_ws = nullptr) {
+                                      int64_t stride_bias = 0, int32_t *prefix_ws = nullptr,
+                                      int64_t prefix_ws_ints = 0) {
   const char *fa = fp8_name(a_type), *fb = fp8_name(b_type);
   if (!fa || !fb)
     return fail(TX_INVALID_ARGUMENT, "%s: operand types must be fp8 (got %d, %d)", what, int(a_type),
@@ -969,14 +974,23 @@ static tx_status dot_fp8_grouped_impl(const char *what, const void *A, tx_dtype 
     return fail(TX_UNSUPPORTED, "%s: a problem's operands exceed 32-bit offsets", what);
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int64_t cus = cu_count();
-  // Groups averaging under 192 rows: the transposed tile (a group's rows on
-  // the tile's 128-wide side, so a 100-row group wastes 28 rows, not 156).
-  const bool trans = grouped && !e.on() && M < 192 * groups;
-  const int64_t tile_rows = trans ? 128 : 256;
+  // Groups averaging under 192 rows take tiles of 128 of their rows (a 100-row
+  // group wastes 28 rows of a tile, not 156) and 256 columns: on the
+  // persistent kernel where it takes the operands (K a whole number (>= 2) of
+  // 128-byte steps, 16-byte aligned C rows), else on the transposed tile,
+  // one workgroup per tile, each paying a pipeline fill and an epilogue.
+  // Before -> persistent, 2048 x 4096 weights: 64 experts, 8192 / 2048 / 256
+  // rows 181 / 174 / 142 -> 157 / 127 / 96 us; 32 x 4096 x 2048, 4096 rows 97
+  // -> 83; 8 x 4096 x 4096, 1024 rows 42 -> 39.
+  const bool pers_ok = grouped && !e.on() && K % 128 == 0 && K >= 256 && N % 8 == 0 && aligned(C, 16) &&
+                       ldc % 8 == 0 && ((M - 1) * ldc + N) * 2 < (int64_t(1) << 31);
+  const bool pers128 = pers_ok && M < 192 * groups;
+  const bool trans = grouped && !e.on() && M < 192 * groups && !pers128;
+  const int64_t tile_rows = trans || pers128 ? 128 : 256;
   const int64_t rt = (M + tile_rows - 1) / tile_rows;
   const int64_t mtiles = grouped ? rt + groups : groups * rt;
-  const bool big = !trans && (grouped ? rt : mtiles) * ((N + 255) / 256) >= cus;
-  const int64_t bn = big || trans ? 256 : 128;  // C columns per tile
+  const bool big = !trans && !pers128 && (grouped ? rt : mtiles) * ((N + 255) / 256) >= cus;
+  const int64_t bn = big || trans || pers128 ? 256 : 128;  // C columns per tile
   const int64_t tiles_n = (N + bn - 1) / bn;
   if (mtiles * tiles_n > INT32_MAX) return fail(TX_UNSUPPORTED, "%s: too many tiles", what);
 
@@ -1005,11 +1019,20 @@ static tx_status dot_fp8_grouped_impl(const char *what, const void *A, tx_dtype 
   ScratchLease pre;  // held until the product is enqueued
   hipFunction_t fn;
   if (grouped) {
+    // The persistent tiles read each m tile's problem from a map after the
+    // prefix, with the groups dealt over the XCDs (the prefix kernel's G^2
+    // ranking stays cheap up to kOrderMaxGroups), where the map fits.
+    const int64_t map_at = (groups + 1 + 3) / 4 * 4, with_map = map_at + 4 * mtiles;
+    const bool map = (pers128 || (big && pers_ok)) && (prefix_ws ? with_map <= prefix_ws_ints : mtiles <= kMapMaxTiles);
     if (prefix_ws) {  // the caller's workspace (the no-allocation entry point)
       q.tile_prefix = prefix_ws;
     } else {
-      TX_TRY(pre.acquire(s, 1, size_t(groups + 1) * sizeof(int32_t)));
+      TX_TRY(pre.acquire(s, 1, size_t(map ? with_map : groups + 1) * sizeof(int32_t)));
       q.tile_prefix = static_cast<int32_t *>(pre.ptr());
+    }
+    if (map) {
+      q.tile_map = q.tile_prefix + map_at;
+      q.dealt = groups > 8 && groups <= kOrderMaxGroups;
     }
     TX_TRY(get_kernel(CodeObject::GemmFp8, "tx_gemm_fp8_grouped_prefix", &fn));
     TX_TRY(launch(fn, 1, 1, 256, s, &q, sizeof q, "tx_gemm_fp8_grouped_prefix"));
@@ -1019,12 +1042,12 @@ static tx_status dot_fp8_grouped_impl(const char *what, const void *A, tx_dtype 
   // persistent kernel (one workgroup per CU walking the real tiles, whose
   // count it reads from the prefix) when K is a whole number (>= 2) of
   // 128-byte steps and C rows are 16-byte aligned.
-  if (grouped && big && !e.on() && K % 128 == 0 && K >= 256 && N % 8 == 0 && aligned(C, 16) && ldc % 8 == 0 &&
-      ((M - 1) * ldc + N) * 2 < (int64_t(1) << 31)) {
-    std::snprintf(kname, sizeof kname, "tx_gemm_fp8_%s_%s_grouped_persist", fa, fb);
+  if (pers128 || (big && pers_ok)) {
+    std::snprintf(kname, sizeof kname, "tx_gemm_fp8_%s_%s_grouped_persist%s", fa, fb, pers128 ? "128" : "");
     TX_TRY(get_kernel(CodeObject::GemmFp8, kname, &fn));
-    return launch(fn, unsigned(std::min<int64_t>(mtiles * tiles_n, cus)), 1, 64 * kPersistWaves, s, &q, sizeof q,
-                  kname);
+    // (128-row tiles: up to 4 column parts each, see gemm_persist.h)
+    return launch(fn, unsigned(std::min<int64_t>(mtiles * tiles_n * (pers128 ? 4 : 1), cus)), 1, 64 * kPersistWaves, s,
+                  &q, sizeof q, kname);
   }
   if (trans) std::snprintf(kname, sizeof kname, "tx_gemm_fp8_%s_%s_grouped_t", fa, fb);
   else std::snprintf(kname, sizeof kname, "tx_gemm_fp8_%s_%s_grouped%s%s", fa, fb, e.on() ? "_epi" : "",
@@ -1034,20 +1057,22 @@ static tx_status dot_fp8_grouped_impl(const char *what, const void *A, tx_dtype 
 }
 
 // The grouped product with an optional caller workspace for the group tile
-// prefix (groups + 1 int32); NULL: the library's stream scratch.
+// prefix and map (prefix_ws_ints int32, at least groups + 1, 16-byte aligned);
+// NULL: the library's stream scratch.
 tx_status dot_fp8_scaled_grouped_ws(const char *what, const void *A, tx_dtype a_type, int64_t lda,
                                     const float *sa, const void *B, tx_dtype b_type, int64_t ldb,
                                     int64_t stride_b, const float *sb, int64_t stride_sb, const float *bias,
                                     int64_t stride_bias, int activation, void *C, tx_dtype c_type,
                                     float c_scale, int64_t ldc, const int32_t *offsets, int64_t groups,
-                                    int64_t M, int64_t N, int64_t K, tx_stream_t stream, int32_t *prefix_ws) {
+                                    int64_t M, int64_t N, int64_t K, tx_stream_t stream, int32_t *prefix_ws,
+                                    int64_t prefix_ws_ints) {
   if (!offsets && groups > 0 && M > 0 && N > 0)
     return fail(TX_INVALID_ARGUMENT, "%s: NULL group offsets", what);
   Epilogue e;
   size_t es;
   TX_TRY(make_epilogue(what, bias, activation, c_type, c_scale, &e, &es));
   return dot_fp8_grouped_impl(what, A, a_type, lda, 0, sa, 0, B, b_type, ldb, stride_b, sb, stride_sb, C,
-                              ldc, 0, offsets, groups, M, N, K, stream, e, es, stride_bias, prefix_ws);
+                              ldc, 0, offsets, groups, M, N, K, stream, e, es, stride_bias, prefix_ws, prefix_ws_ints);
 }
 
 static tx_status dot_fp8_scaled_grouped(const void *A, tx_dtype a_type, int64_t lda, const float *sa,
@@ -1058,7 +1083,7 @@ static tx_status dot_fp8_scaled_grouped(const void *A, tx_dtype a_type, int64_t 
                                         int64_t M, int64_t N, int64_t K, tx_stream_t stream) {
   return dot_fp8_scaled_grouped_ws("tx_dot_fp8_scaled_grouped", A, a_type, lda, sa, B, b_type, ldb,
                                        stride_b, sb, stride_sb, bias, stride_bias, activation, C, c_type,
-                                       c_scale, ldc, offsets, groups, M, N, K, stream, nullptr);
+                                       c_scale, ldc, offsets, groups, M, N, K, stream, nullptr, 0);
 }
 
 static tx_status gemv_fp8_dequant(const void *x, int64_t ldx, const void *W, tx_dtype w_type,

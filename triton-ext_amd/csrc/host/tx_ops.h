@@ -61,7 +61,8 @@ tx_status dot_fp8_scaled_grouped_ws(const char *what, const void *A, tx_dtype a_
                                     int64_t stride_b, const float *sb, int64_t stride_sb, const float *bias,
                                     int64_t stride_bias, int activation, void *C, tx_dtype c_type,
                                     float c_scale, int64_t ldc, const int32_t *offsets, int64_t groups,
-                                    int64_t M, int64_t N, int64_t K, tx_stream_t stream, int32_t *prefix_ws);
+                                    int64_t M, int64_t N, int64_t K, tx_stream_t stream, int32_t *prefix_ws,
+                                    int64_t prefix_ws_ints);
 
 #define TX_TRY(expr)                      \
   do {                                    \

@@ -55,6 +55,9 @@ TX_GEMM_FP8_FAST(e5m2, e4m3fn, EL_E5M2, EL_E4M3)
   }                                                                                                         \
   TX_KERNEL void __launch_bounds__(256) tx_gemm_fp8_##FA##_##FB##_grouped_persist(const tx_grouped_args q) { \
     gemm_persist<GemmCfg<ELA, ELB, 256, 256, 2, 2, 16>, OUT_BF16, true>(q.g, &q);                            \
+  }                                                                                                         \
+  TX_KERNEL void __launch_bounds__(256) tx_gemm_fp8_##FA##_##FB##_grouped_persist128(const tx_grouped_args q) { \
+    gemm_persist<GemmCfg<ELA, ELB, 256, 256, 2, 2, 16>, OUT_BF16, true, false, false, 128, 256>(q.g, &q);    \
   }
 
 TX_GEMM_FP8_PERSIST(e4m3fn, e4m3fn, EL_E4M3, EL_E4M3)
@@ -118,32 +121,100 @@ TX_KERNEL void __launch_bounds__(256) tx_gemm_fp8_epilogue(const tx_gemm_args a)
 // workgroup per (problem, tile), no K split.
 //
 // Tile prefix of a grouped product: one workgroup scans the groups' m-tile
-// counts ceil(rows / 256) in chunks of 256 (rows from the clamped offsets).
+// counts ceil(rows / tile_rows) in chunks of 256 (rows from the clamped
+// offsets) into tile_prefix[0 .. groups], and with q.tile_map writes each m
+// tile's problem and rows beside it (one 16-byte scalar load in the product
+// instead of a search of dependent ones).
+// q.dealt (at most kOrderMax groups): the map holds the groups by falling tile
+// count, dealt to 8 runs back and forth, one run after the other.  Each
+// XCD's eighth of the tiles then holds about an eighth of the experts: in the
+// caller's order one XCD can get all tiles of one large expert (whose weights
+// it reads once) and another as many experts of one tile each, and the
+// kernel waits for the XCD that streams the most weights.
+// (tile_prefix[groups], the total, is the same either way; the entries before
+// it are then not used.)  64 skewed experts, 8192 x 2048 x 4096, 96 m tiles: the
+// product 161 us on the transposed 256 x 128 tile, 127 us on the 128 x 256
+// persistent one with its tiles dealt.  Offsets that are not nondecreasing can give more m
+// tiles than the mtiles the map has room for: the map is then not written and
+// the product, which sees the same total, searches the prefix.
+constexpr int kOrderMax = 512;
 TX_KERNEL void __launch_bounds__(256) tx_gemm_fp8_grouped_prefix(const tx_grouped_args q) {
-  __shared__ int sc[256];
+  __shared__ int wave_sum[4], cnt[kOrderMax], run_cnt[kOrderMax + 8], run_of[kOrderMax + 8];
   const int t = threadIdx.x;
   const int total = q.g.M;
-  int carry = 0;
+  auto rows_of = [&](int p, int *r0) {
+    const int r1 = min(max(q.offsets[p + 1], 0), total);
+    *r0 = min(max(q.offsets[p], 0), r1);
+    return r1 - *r0;
+  };
+  auto tiles_of = [&](int p) {
+    int r0;
+    return (rows_of(p, &r0) + q.tile_rows - 1) / q.tile_rows;
+  };
+  const int run = (q.groups + 7) / 8;
+  bool dealt = q.dealt != 0;
   if (t == 0) q.tile_prefix[0] = 0;
-  for (int base = 0; base < q.groups; base += 256) {
-    const int p = base + t;
-    int c = 0;
-    if (p < q.groups) {
-      const int r1 = min(max(q.offsets[p + 1], 0), total);
-      const int r0 = min(max(q.offsets[p], 0), r1);
-      c = (r1 - r0 + q.tile_rows - 1) / q.tile_rows;
-    }
-    sc[t] = c;
+  if (dealt) {
+    const int places = 8 * run;
+    for (int p = t; p < q.groups; p += 256) cnt[p] = tiles_of(p);
+    for (int i = t; i < places; i += 256) run_cnt[i] = 0;
     __syncthreads();
-    for (int d = 1; d < 256; d *= 2) {  // inclusive scan
-      const int v = t >= d ? sc[t - d] : 0;
+    for (int p = t; p < q.groups; p += 256) {
+      const int mine = cnt[p];
+      int rank = 0;
+      for (int j = 0; j < q.groups; ++j) rank += cnt[j] > mine || (cnt[j] == mine && j < p);
+      const int row = rank >> 3, col = rank & 7, i = ((row & 1) ? 7 - col : col) * run + row;
+      run_cnt[i] = mine;
+      run_of[i] = p;
+    }
+    __syncthreads();
+  }
+  int carry, places;
+  for (;;) {
+    carry = 0;
+    places = dealt ? 8 * run : q.groups;
+    for (int base = 0; base < places; base += 256) {
+      const int i = base + t;
+      const int c = i >= places ? 0 : dealt ? run_cnt[i] : tiles_of(i);
+      int incl = c;  // inclusive scan: within the wavefront, then over the four
+#pragma unroll
+      for (int d = 1; d < 64; d *= 2) {
+        const int v = __shfl_up(incl, d);
+        if ((t & 63) >= d) incl += v;
+      }
+      if ((t & 63) == 63) wave_sum[t >> 6] = incl;
       __syncthreads();
-      sc[t] += v;
+      int all = 0;
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        if (w == t >> 6) incl += all;
+        all += wave_sum[w];
+      }
+      if (i < places) {
+        if (dealt) run_cnt[i] = carry + incl - c;  // first m tile of the place
+        else q.tile_prefix[i + 1] = carry + incl;
+      }
+      carry += all;
       __syncthreads();
     }
-    if (p < q.groups) q.tile_prefix[p + 1] = carry + sc[t];
-    carry += sc[255];
-    __syncthreads();
+    if (!dealt || carry <= q.mtiles) break;
+    dealt = false;
+  }
+  if (dealt && t == 0) q.tile_prefix[q.groups] = carry;
+  if (!q.tile_map || carry > q.mtiles) return;
+  __threadfence_block();
+  __syncthreads();
+  for (int vm = t; vm < carry; vm += 256) {
+    int lo = 0, hi = places - 1;  // the last place whose first m tile is <= vm
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if ((dealt ? run_cnt[mid] : q.tile_prefix[mid]) <= vm) lo = mid;
+      else hi = mid - 1;
+    }
+    const int p = dealt ? run_of[lo] : lo;
+    int r0;
+    const int rows = rows_of(p, &r0);
+    reinterpret_cast<int4 *>(q.tile_map)[vm] = int4{p, r0, rows, vm - (dealt ? run_cnt[lo] : q.tile_prefix[lo])};
   }
 }
 

@@ -1,16 +1,16 @@
 // Persistent 4-wavefront GEMM for aligned operands whose K is a whole number
 // of 128-byte steps (KTAIL, 16-bit operands: rows 4-byte aligned, any K of
 // at least two steps, read as fast::KTail describes, and C rows of any
-// alignment): one workgroup per CU walks its share of the BT x BT tiles
-// (BT = 256; 128 or 64 for products with fewer 256 x 256 / 128 x 128 tiles
+// alignment): one workgroup per CU walks its share of the BM x BN tiles
+// (256 x 256; 128 x 128 or 64 x 64 for products with fewer 256 x 256 / 128 x 128 tiles
 // than CUs),
 // and the LDS-DMA pipeline of gemm_fast.h runs as one continuous
 // stream of (tile, K step) pairs, so the first steps of the next tile are
 // loaded while the current one finishes and no tile pays a pipeline fill.
 //
 // Layout per workgroup: 4 wavefronts (one per SIMD) in a 2 x 2 grid, each
-// owning a BT / 2 square block of the tile; its accumulator blocks of 16 x 16
-// (BT = 256: 64 blocks, 256 registers) live in AGPRs.  Against the
+// owning a quarter of the tile; its accumulator blocks of 16 x 16
+// (256 x 256: 64 blocks, 256 registers) live in AGPRs.  Against the
 // 8-wavefront tile this reads a third less from LDS per MFMA, which the power-
 // limited clock turns into speed.
 //
@@ -21,15 +21,15 @@
 // loops on N(0,1) operands sustain 2025 against 1765 TFLOP/s (bf16) and 4360
 // against 3970 (fp8).  In this kernel (32 x 32 -> 16 x 16, same box): fp16
 // 4096^3 row-major B 110 -> 107 us (clock 1.75 -> 2.00 GHz, MFMA busy 64 ->
-// 60%), bf16 8192^3 764 -> 721 us, 2048^3 (BT = 128) 22.8 -> 21.6 us, fp8
+// 60%), bf16 8192^3 764 -> 721 us, 2048^3 (128 x 128) 22.8 -> 21.6 us, fp8
 // 8192^3 371 -> 359 us.  Without the LDS-DMA stream (timing only) these take
 // 93, 628, 19.5 and 300 us: what binds them now is that stream's power and
 // its delivery, not MFMA issue (staggering reads and loads, or forcing the
 // accumulators in place, moves nothing beyond 1%).
 //
-// The K loop is that of gemm_fast_tile_at (ring of 5 LDS slots of BT x 128 bytes,
-// B of step s+2 and A of step s+3 loaded during the second half of step s; BT
-// below 256: 5 or 8 stages of a whole step, both of step s+5 or s+8,
+// The K loop is that of gemm_fast_tile_at (ring of 5 LDS slots of 256 x 128 bytes,
+// B of step s+2 and A of step s+3 loaded during the second half of step s; smaller
+// tiles: D stages of a whole step, both of step s+D,
 // fragments one 64-byte half ahead in registers, one barrier per step), with
 // s counting steps over all tiles of the workgroup.  Each operand's loads go
 // through a buffer resource for the tile they belong to: base at the tile's
@@ -48,8 +48,8 @@
 // loads of step s+3 are deferred so that their LDS slot stages the output:
 // per 32 x 32 block the accumulators are scaled, rounded to bf16 / fp16
 // (RNE), and lanes l and l + 32 exchange halves (v_permlane32_swap); each
-// wave writes its 32 x BT / 2 block to its own quarter of that slot, reads
-// back whole rows (BT = 256: 4 of 256 bytes) per instruction and stores them
+// wave writes its 32 x BN / 2 block to its own quarter of that slot, reads
+// back whole rows (BN = 256: 4 of 256 bytes) per instruction and stores them
 // through a buffer
 // resource for C (stores past M / N are dropped).  OUT_F32 (tt.dot with its
 // accumulator operand): D = A.B + C in fp32 is written straight from the
@@ -134,16 +134,17 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rsrc(const void *base, in
 // B + p stride_b and scale_b + p stride_sb.
 //
 // BKN: B is row-major K x N (16-bit operands, K a whole number of steps).  A
-// step of B is then 64 K rows of the tile's BT columns (2 BT bytes each),
+// step of B is then 64 K rows of the tile's BN columns (2 BN bytes each),
 // DMA'd into a K-major slot whose 16-byte chunk c of K row k sits at
-// c ^ kn_swz(k mod 4, 2 BT), and each B fragment is two transposing LDS reads
+// c ^ kn_swz(k, 2 BN), and each B fragment is two transposing LDS reads
 // (ds_read_b64_tr_b16): in each 16-lane group, lane s reads 4 columns at K
 // row s / 4 and lane d receives column d's 4 K values, the register layout
 // the MFMA takes.  The swizzle keeps a group's 4 rows x 2 chunks on 8
 // distinct 16-byte bank groups of 128 bytes, and a 32-lane half's 4 rows x
 // 4 chunks on 16 of 256 bytes (for 128-byte rows, two to 256 bytes of
 // banks: on 8 of 128 and on 16 half-row positions).
-template <class C, int OUT = OUT_BF16, bool GROUPED = false, bool KTAIL = false, bool BKN = false, int BT = 256>
+template <class C, int OUT = OUT_BF16, bool GROUPED = false, bool KTAIL = false, bool BKN = false, int BM = 256,
+          int BN = BM>
 __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_grouped_args *q = nullptr) {
   using namespace fast;
   static_assert(OUT == OUT_BF16 || (OUT == OUT_F16 && !C::FP8) || (OUT == OUT_F32 && !C::FP8),
@@ -151,33 +152,49 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
   constexpr bool F32 = OUT == OUT_F32;
   static_assert(!KTAIL || (!C::FP8 && !GROUPED), "ragged K: 16-bit operands, one product");
   static_assert(!BKN || (!C::FP8 && !GROUPED && !KTAIL), "row-major B: 16-bit operands, whole K steps");
-  static_assert(BT == 256 || BT == 128 || BT == 64, "tile 256, 128 or 64 square");
+  static_assert(BM == BN ? BM == 256 || BM == 128 || BM == 64 : BM == 128 && BN == 256 && GROUPED,
+                "tile 256, 128 or 64 square; grouped also 128 x 256");
   constexpr int NW = persist::kWaves;
-  constexpr int TM = BT / 2, TN = BT / 2, FM = TM / 16, FN = TN / 16;
+  constexpr int TM = BM / 2, TN = BN / 2, FM = TM / 16, FN = TN / 16;
   // MFMAs of a K step's half (16-bit: K half h; fp8: half of the columns)
   constexpr int NM = C::FP8 ? FM * FN / 2 : FM * FN, NF = FM + FN, NR = NF;
-  static_assert(!C::FP8 || BT == 256, "fp8: the 256 x 256 tile");
-  constexpr int SB = BT * kStep;  // one operand of one K step
-  constexpr int BLKA = SB / 1024 / NW, BLKB = BLKA, ND = BLKA + BLKB;
+  static_assert(!C::FP8 || BN == 256, "fp8: 256 columns");
+  constexpr int SBA = BM * kStep, SBB = BN * kStep;  // one operand of one K step
+  constexpr int BLKA = SBA / 1024 / NW, BLKB = SBB / 1024 / NW, ND = BLKA + BLKB;
   constexpr int RW = NM >= 2 ? NM / 2 : 1;
-  // Ring: BT = 256, 5 slots of one operand of one step (B two steps ahead, A
+  // Ring: 256 x 256, 5 slots of one operand of one step (B two steps ahead, A
   // three); smaller tiles, whose step is a fraction of the time a load
   // takes to arrive, D stages of a step's A and B slots, both loaded D steps
-  // ahead (160 and 128 KiB): against the 5-slot ring fp16 640 x 2000 x 3968
-  // (BT = 64) 51.7 -> 33.0 us, 2304 x 2304 x 4096 (BT = 128) 68.1 -> 59.7.
-  constexpr bool STG = BT < 256;
-  constexpr int D = BT == 128 ? 5 : 8, NSLOT = STG ? 2 * D : kSlots;
+  // ahead (128 x 128: 5, 160 KiB; 64 x 64: 8, 128 KiB): against the 5-slot ring
+  // fp16 640 x 2000 x 3968 (64 x 64) 51.7 -> 33.0 us, 2304 x 2304 x 4096 (128
+  // x 128) 68.1 -> 59.7.  128 x 256: 3 stages, 144 KiB.
+  constexpr bool STG = BM < 256;
+  constexpr int D = BM != BN ? 3 : BM == 128 ? 5 : 8, STAGE = SBA + SBB;
+  constexpr int kLds = STG ? D * STAGE : kSlots * SBA;
+  // The epilogue stages its output in the larger slot (A's if equal), whose
+  // loads of the last step wait until it is done: operand op_st.
+  constexpr int op_st = BN > BM ? 1 : 0, kLastLoads = op_st == 0 ? BLKB : BLKA;
   constexpr bool ROWCOL = C::FP8;
   // BKN: bytes of a K row of the B tile, and K rows per 1 KiB DMA block
-  constexpr int KRB = 2 * BT, RPB = 1024 / KRB, CPR = KRB / 16;
-  __shared__ __attribute__((aligned(1024))) uint8_t lds[NSLOT * SB];
+  constexpr int KRB = 2 * BN, RPB = 1024 / KRB, CPR = KRB / 16;
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[kLds];
 
   // m tiles: the grouped product's real count is only on the device
   const int tiles_m = GROUPED ? q->tile_prefix[q->groups] : a.tiles_m;
+  const bool use_map = GROUPED && q->tile_map && tiles_m <= q->mtiles;
   const int total = tiles_m * a.tiles_n;
   const int G = int(gridDim.x);
   const int w = int(blockIdx.x);
-  const int T = w < total ? (total - w + G - 1) / G : 0;  // tiles of this workgroup
+  // COLS: the tiles of a last round that would leave at least half of the
+  // workgroups idle are cut into 2 or 4 column parts, one to a workgroup.  The
+  // grouped product streams weights from HBM, and a few whole tiles alone on
+  // the chip take as long as a full round of them.  (The MFMAs of the columns
+  // outside a part run on zeros.)
+  constexpr bool COLS = GROUPED && BM < 256;
+  const int whole = COLS ? total / G * G : total, over = total - whole;
+  const int parts = !COLS || over == 0 ? 1 : over * 4 <= G ? 4 : over * 2 <= G ? 2 : 1;
+  const int units = whole + over * parts;
+  const int T = w < units ? (units - w + G - 1) / G : 0;  // tiles (or parts) of this workgroup
   if (T == 0) return;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -197,9 +214,9 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
   // filling chunk position p mod CPR of row + p / CPR.  The swizzle goes by
   // the row's low two bits and bit 3, so block j shares the lane offsets of
   // block kn_rep(j), kept at kn_var(j).
-  constexpr auto kn_rep = [](int j) constexpr { return BT == 256 ? (j & 1) + 4 * (j >> 2) : BT == 128 ? j & ~1 : j; };
-  constexpr auto kn_var = [](int j) constexpr { return BT == 256 ? (j & 1) + 2 * (j >> 2) : BT == 128 ? j >> 1 : j; };
-  constexpr int NVB = BKN && BT == 256 ? 4 : 2;
+  constexpr auto kn_rep = [](int j) constexpr { return BN == 256 ? (j & 1) + 4 * (j >> 2) : BN == 128 ? j & ~1 : j; };
+  constexpr auto kn_var = [](int j) constexpr { return BN == 256 ? (j & 1) + 2 * (j >> 2) : BN == 128 ? j >> 1 : j; };
+  constexpr int NVB = BKN && BN == 256 ? 4 : 2;
   uint32_t vo[2][NVB];
 #pragma unroll
   for (int e = 0; e < 2; ++e) vo[0][e] = uint32_t(8 * (BLKA * wave + e) + (lane >> 3)) * lda_b + kch[e];
@@ -237,12 +254,21 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
     const uint8_t *A, *B;
     uint8_t *out;  // C
     const float *sa, *sb;
-    int rows, tm, tn;
+    int rows, tm, p;
+    int n0, nend;  // columns n0 .. min(nend, n0 + BN) - 1
   };
   auto desc = [&](int t) {
     TileDesc d;
-    int vm;
-    tile_coords(w + t * G, a.tiles_n, tiles_m, min(8, a.tiles_n), &d.tn, &vm);  // transposed grid
+    int vm, tn;
+    const int u = w + t * G;
+    const int tile = u < whole ? u : whole + (u - whole) / parts;
+    tile_coords(tile, a.tiles_n, tiles_m, min(8, a.tiles_n), &tn, &vm);  // transposed grid
+    d.n0 = tn * BN;
+    d.nend = a.N;
+    if (COLS && u >= whole) {
+      d.n0 += (u - whole) % parts * (BN / parts);
+      d.nend = min(d.nend, d.n0 + BN / parts);
+    }
     d.A = static_cast<const uint8_t *>(a.A);
     d.B = static_cast<const uint8_t *>(a.B);
     d.out = static_cast<uint8_t *>(a.C);
@@ -250,23 +276,41 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
     d.sb = a.scale_b;
     d.rows = a.M;
     d.tm = vm;
+    d.p = 0;
     if constexpr (GROUPED) {
-      const int32_t *Tp = q->tile_prefix;
-      int lo = 0, hi = q->groups - 1;  // the last problem p with Tp[p] <= vm
-      while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (Tp[mid] <= vm) lo = mid;
-        else hi = mid - 1;
+      int p, r0;
+      if (use_map) {
+        const int4 e = reinterpret_cast<const int4 *>(q->tile_map)[vm];
+        p = e.x;
+        r0 = e.y;
+        d.rows = e.z;
+        d.tm = e.w;
+      } else {
+        const int32_t *Tp = q->tile_prefix;
+        int lo = 0, hi = q->groups - 1;  // the last problem p with Tp[p] <= vm
+        while (lo < hi) {
+          const int mid = (lo + hi + 1) >> 1;
+          if (Tp[mid] <= vm) lo = mid;
+          else hi = mid - 1;
+        }
+        p = lo;
+        const int r1 = min(max(q->offsets[p + 1], 0), a.M);
+        r0 = min(max(q->offsets[p], 0), r1);
+        d.rows = r1 - r0;
+        d.tm = vm - Tp[lo];
       }
-      const int r1 = min(max(q->offsets[lo + 1], 0), a.M);
-      const int r0 = min(max(q->offsets[lo], 0), r1);
+      // (uniform, but loaded through vector memory: buffer resources made
+      // from vector registers would turn every operand load into a loop)
+      p = __builtin_amdgcn_readfirstlane(p);
+      r0 = __builtin_amdgcn_readfirstlane(r0);
+      d.rows = __builtin_amdgcn_readfirstlane(d.rows);
+      d.tm = __builtin_amdgcn_readfirstlane(d.tm);
       d.A += int64_t(r0) * a.lda;
-      d.B += int64_t(lo) * q->stride_b;
+      d.B += int64_t(p) * q->stride_b;
       d.out += int64_t(r0) * a.ldc * 2;
       d.sa += r0;
-      d.sb += int64_t(lo) * q->stride_sb;
-      d.rows = r1 - r0;
-      d.tm = vm - Tp[lo];
+      d.sb += int64_t(p) * q->stride_sb;
+      d.p = p;
     }
     return d;
   };
@@ -274,43 +318,55 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
   // Load cursor of one operand: the step it is at and the buffer resource of
   // that step's tile (an empty range past the last tile).  Steps advance
   // one at a time.
+  // ROT: a tile's K steps run from a start of its own (by expert, spread over
+  // K, so tiles that share rows of A or B stay in step) and wrap around: kp
+  // is the step's place in K, k its number.  Experts' weights are read from
+  // HBM, and with a row pitch of a power of two the same K step of every row
+  // sits on the same few channels: 64 experts x 2048 x 4096, 256 rows in all
+  // (weights alone), 131 us in step, 97 us rotated.
+  constexpr bool ROT = GROUPED && BM < 256;
   struct Cursor {
-    int t, k;
+    int t, k, kp;
     __amdgpu_buffer_rsrc_t rs;
   };
   auto set_tile = [&](Cursor &c, auto op_tag) {
     constexpr int op = decltype(op_tag)::value;
+    c.kp = 0;
     if (c.t < T) {
       const TileDesc d = desc(c.t);
+      if constexpr (ROT) c.kp = int(__umulhi(uint32_t(d.p) * 2654435769u, uint32_t(KS)));
       if constexpr (BKN && op == 1) {
-        // columns BT tn .. of all K rows, the range ending at the last
+        // columns n0 .. of all K rows, the range ending at the last
         // row's last column (columns past N in earlier rows read that
         // row's padding or the next row: their products are not stored)
-        c.rs = make_rsrc(d.B + int64_t(d.tn) * KRB, uint32_t(a.K - 1) * ldb_b + uint32_t(a.N - d.tn * BT) * 2u);
+        c.rs = make_rsrc(d.B + int64_t(d.n0) * 2, uint32_t(a.K - 1) * ldb_b + uint32_t(a.N - d.n0) * 2u);
       } else {
-        c.rs = op == 0 ? persist::tile_rsrc<BT>(d.A, d.tm * BT, d.rows, lda_b, kb_end)
-                       : persist::tile_rsrc<BT>(d.B, d.tn * BT, a.N, ldb_b, kb_end);
+        c.rs = op == 0                   ? persist::tile_rsrc<BM>(d.A, d.tm * BM, d.rows, lda_b, kb_end)
+               : COLS && d.n0 >= d.nend ? make_rsrc(a.B, 0u)
+                                         : persist::tile_rsrc<BN>(d.B, d.n0, d.nend, ldb_b, kb_end);
       }
     } else {
       c.rs = make_rsrc(op == 0 ? a.A : a.B, 0u);
     }
   };
   auto advance = [&](Cursor &c, auto op_tag) {
+    ++c.kp;
+    if (ROT && c.kp == KS) c.kp = 0;
     if (++c.k == KS) {
       c.k = 0;
       ++c.t;
       set_tile(c, op_tag);
     }
   };
-  auto load_op = [&](const Cursor &c, int slot, auto op_tag, auto j_tag) {
+  auto load_op = [&](const Cursor &c, int base, auto op_tag, auto j_tag) {
     constexpr int op = decltype(op_tag)::value, j = decltype(j_tag)::value;
     constexpr int blk = op == 0 ? BLKA : BLKB;
-    uint8_t *dst = lds + slot * SB + (blk * wave + j) * 1024;
+    uint8_t *dst = lds + base + (blk * wave + j) * 1024;
     const bool lk = KTAIL && c.k == KS - 1;  // (c.k >= 1 there)
     constexpr int var = BKN && op == 1 ? kn_var(j) : j & 1;
     constexpr int past = BKN && op == 1 ? j - kn_rep(j) : j & ~1;  // blocks past the one of those offsets
     __builtin_amdgcn_raw_ptr_buffer_load_lds(c.rs, (lds_void *)dst, 16, lk ? vl[op][j & 1] : vo[op][var],
-                                             uint32_t(c.k) * kstep_b[op] + uint32_t(past) * ld8[op] -
+                                             uint32_t(c.kp) * kstep_b[op] + uint32_t(past) * ld8[op] -
                                                  (lk ? 16u : 0u),
                                              0, 0);
   };
@@ -342,8 +398,8 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
     }
   }
   txd::i32x4 fr[NF][2];
-  // Read piece x of fragment f from the step in slots slot_a, slot_b.
-  auto read_piece = [&](int slot_a, int slot_b, auto f_tag, auto x_tag) {
+  // Read piece x of fragment f of the step at LDS bytes base_a, base_b.
+  auto read_piece = [&](int base_a, int base_b, auto f_tag, auto x_tag) {
     constexpr int f = decltype(f_tag)::value, x = decltype(x_tag)::value;
     if constexpr (BKN && f >= FM) {
       // Inline asm: the compiler puts a vmcnt(0) (a drain of every operand
@@ -351,7 +407,7 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
       // LDS-DMA load is pending.  Its results are waited for explicitly:
       // kn_wait in the K step's first half, the barrier in the second.
       constexpr int c0 = 32 * x * KRB;
-      const uint32_t addr = lds_base + uint32_t(slot_b * SB + bko[f - FM]);
+      const uint32_t addr = lds_base + uint32_t(base_b + bko[f - FM]);
       txd::u32x2 lo, hi;
       asm volatile("ds_read_b64_tr_b16 %0, %2 offset:%3\n\tds_read_b64_tr_b16 %1, %2 offset:%4"
                    : "=&v"(lo), "=&v"(hi)
@@ -359,16 +415,16 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
                    : "memory");
       fr[f][x] = txd::i32x4{int(lo[0]), int(lo[1]), int(hi[0]), int(hi[1])};
     } else {
-      const uint8_t *Sp = lds + (f < FM ? slot_a : slot_b) * SB;
+      const uint8_t *Sp = lds + (f < FM ? base_a : base_b);
       const int byte = f < FM ? ro[0][x] + 2048 * f : ro[1][x] + 2048 * (f - FM);
       fr[f][x] = *reinterpret_cast<const txd::i32x4 *>(Sp + byte);
     }
   };
   // Read r of K half h (16-bit), in the order the MFMAs consume them: A0, B0,
   // A1 .. A(FM-1), B1 .. B(FN-1).
-  auto read = [&](int slot_a, int slot_b, auto h_tag, auto r_tag) {
+  auto read = [&](int base_a, int base_b, auto h_tag, auto r_tag) {
     constexpr int o = decltype(r_tag)::value, f = o == 0 ? 0 : o == 1 ? FM : o <= FM ? o - 1 : o;
-    read_piece(slot_a, slot_b, std::integral_constant<int, f>{}, h_tag);
+    read_piece(base_a, base_b, std::integral_constant<int, f>{}, h_tag);
   };
   // LDS operations of reads 0 .. r - 1 of a K half (BKN: two per B block).
   constexpr auto read_ops = [](int r) constexpr { return r + (r >= 2 ? 1 : 0) + (r > FM + 1 ? r - FM - 1 : 0); };
@@ -392,7 +448,7 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
     persist::mfma16<C>(acc[fn][fm], fr[FM + fn], fr[fm], h);
     // (kept in its AGPRs: left alone the ragged-K variant rotates blocks
     // through VGPRs and spills 26 of them, and the fp32 one copies them)
-    if constexpr (KTAIL || (F32 && BT < 256)) asm volatile("" : "+a"(acc[fn][fm]));
+    if constexpr (KTAIL || (F32 && BM < 256)) asm volatile("" : "+a"(acc[fn][fm]));
   };
   using H0 = std::integral_constant<int, 0>;
   using H1 = std::integral_constant<int, 1>;
@@ -404,9 +460,9 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
   set_tile(ca, OpA{});
   set_tile(cb, OpB{});
   static_for<STG ? D : 2>([&](auto st) {
-    constexpr int sl = 2 * decltype(st)::value;
-    static_for<BLKA>([&](auto j) { load_op(ca, sl, OpA{}, j); });
-    static_for<BLKB>([&](auto j) { load_op(cb, sl + 1, OpB{}, j); });
+    constexpr int la = decltype(st)::value * (STG ? STAGE : 2 * SBA), lb = la + SBA;
+    static_for<BLKA>([&](auto j) { load_op(ca, la, OpA{}, j); });
+    static_for<BLKB>([&](auto j) { load_op(cb, lb, OpB{}, j); });
     advance(ca, OpA{});
     advance(cb, OpB{});
   });
@@ -414,23 +470,23 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
     wait_and_barrier<(D - 1) * ND>();
   } else {
     // (next B load: step 2, next A load: step 3)
-    static_for<BLKA>([&](auto j) { load_op(ca, 4, OpA{}, j); });
+    static_for<BLKA>([&](auto j) { load_op(ca, 4 * SBA, OpA{}, j); });
     advance(ca, OpA{});
     wait_and_barrier<2 * BLKA + BLKB>();
   }
   // The fragments a step starts with: 16-bit, its first K half; fp8, all of A
   // and the first two B blocks.
-  auto read_start = [&](int slot_a, int slot_b) {
+  auto read_start = [&](int base_a, int base_b) {
     if constexpr (C::FP8) {
       static_for<FM + 2>([&](auto f) {
-        read_piece(slot_a, slot_b, f, H0{});
-        read_piece(slot_a, slot_b, f, H1{});
+        read_piece(base_a, base_b, f, H0{});
+        read_piece(base_a, base_b, f, H1{});
       });
     } else {
-      static_for<NR>([&](auto r) { read(slot_a, slot_b, H0{}, r); });
+      static_for<NR>([&](auto r) { read(base_a, base_b, H0{}, r); });
     }
   };
-  read_start(0, 1);
+  read_start(0, SBA);
 
   // One K step: half 0 (reads of the rest of the step's fragments), barrier,
   // half 1 (loads of B s+2 and A s+3, reads of the first fragments of step
@@ -442,16 +498,16 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
   // FIRST: the tile's first step
   // (MFMAs from a zero accumulator); VM: loads and stores allowed in flight
   // at the barrier (the next step's operands are older than the last VM);
-  // LAST: the tile's last step, whose A s+3 loads wait until after the
-  // epilogue (their slot stages the output tile), as do the reads of the
+  // LAST: the tile's last step, whose loads into the staging slot (op_st)
+  // wait until after the epilogue, as do the reads of the
   // next step's first half (their registers hold the column scales).
-  int sa = 0, sb = 1;
+  int sa = 0, sb = SBA;  // LDS bytes of step s's A and B
   auto step = [&](auto first_tag, auto vm_tag, auto last_tag) {
     constexpr int VM = decltype(vm_tag)::value;
     constexpr bool LAST = decltype(last_tag)::value;
-    // slots of step s+1, and those the loads go into (free after the barrier)
-    const int na = STG ? (sa == 2 * (D - 1) ? 0 : sa + 2) : sa >= 3 ? sa - 3 : sa + 2;
-    const int nb = STG ? na + 1 : sb >= 3 ? sb - 3 : sb + 2;
+    // those of step s+1, and of the loads (step s's, free after the barrier)
+    const int na = STG ? (sa == (D - 1) * STAGE ? 0 : sa + STAGE) : sa >= 3 * SBA ? sa - 3 * SBA : sa + 2 * SBA;
+    const int nb = STG ? na + SBA : sb >= 3 * SBA ? sb - 3 * SBA : sb + 2 * SBA;
     const int la = STG ? sa : sb, lb = STG ? sb : sa;
     const bool clear = KTAIL && LAST && kt.cp < 8;
     if (clear) persist::ktail_clear<NF>(fr, 0, fg, kt);
@@ -463,8 +519,8 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
       mma(H0{}, Fn{}, Fm{}, first_tag);
       __builtin_amdgcn_sched_barrier(0);
       if constexpr (C::FP8) {
-        // B blocks 2 .. FN-1, two pieces each
-        constexpr int n = 2 * (FN - 2), r0 = spread_lo(i, n, 2 * n), r1 = spread_hi(i, n, 2 * n);
+        // B blocks 2 .. FN-1, two pieces each, over three quarters of the MFMAs
+        constexpr int n = 2 * (FN - 2), r0 = spread_lo(i, n, NM * 3 / 4), r1 = spread_hi(i, n, NM * 3 / 4);
         static_for<r1 - r0>([&](auto R) {
           constexpr int r = r0 + decltype(R)::value;
           read_piece(sa, sb, std::integral_constant<int, FM + 2 + r / 2>{}, std::integral_constant<int, r % 2>{});
@@ -498,8 +554,11 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
       constexpr int d0 = nd(i), d1 = nd(i + 1);
       static_for<d1 - d0>([&](auto D) {
         constexpr int d = d0 + decltype(D)::value;
-        if constexpr (d < BLKB) load_op(cb, lb, OpB{}, std::integral_constant<int, d>{});
-        else if constexpr (!LAST) load_op(ca, la, OpA{}, std::integral_constant<int, d - BLKB>{});
+        if constexpr (d < BLKB) {
+          if constexpr (!LAST || op_st == 0) load_op(cb, lb, OpB{}, std::integral_constant<int, d>{});
+        } else if constexpr (!LAST || op_st == 1) {
+          load_op(ca, la, OpA{}, std::integral_constant<int, d - BLKB>{});
+        }
       });
       if constexpr (!LAST && C::FP8) {
         // A block i / HF after its last MFMA (the second piece one MFMA on),
@@ -517,8 +576,8 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
       }
       __builtin_amdgcn_sched_barrier(0);
     });
-    advance(cb, OpB{});
-    if constexpr (!LAST) advance(ca, OpA{});
+    if constexpr (!LAST || op_st == 0) advance(cb, OpB{});
+    if constexpr (!LAST || op_st == 1) advance(ca, OpA{});
     sa = na;
     sb = nb;
   };
@@ -534,11 +593,12 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
   constexpr int SRB = 2 * TN, CH = SRB / 16, SPI = 64 / CH;
   constexpr int kEpiStores = F32 ? FM * FN : FM / 2 * (32 / SPI);
   constexpr int kAfterEpi = kAhead + kEpiStores + (STG ? 0 : BLKB - BLKA);
+  static_assert(32 * SRB * NW <= (op_st == 0 ? SBA : SBB), "the staging fits its slot");
   using VmAfterEpi = std::integral_constant<int, (kAfterEpi < 64 ? kAfterEpi : 63)>;
   // Scale loads issued before the last step (row scales, column-scale
   // vectors) that its barrier leaves in flight with the step's own A loads.
   // F32: the tile's accumulator operand (C), 4 columns per load, is read in
-  // batches of FB row blocks, 16 loads (BT = 64: 4; KTAIL, short of registers:
+  // batches of FB row blocks, 16 loads (64 x 64: 4; KTAIL, short of registers:
   // 8) each, the first before the last step.
   constexpr int FB = FM < 4 ? FM : KTAIL ? 1 : 16 / FN, NB = FM / FB;
   constexpr int kScaleLoads = ROWCOL ? FM + FN : F32 ? FB * FN : 0;
@@ -546,18 +606,18 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
   static_assert(kAhead + kScaleLoads < 64, "vmcnt range");
 
   // Staging: wave w owns bytes 32 SRB w .. + 32 SRB of the slot its last
-  // step's A s+3 loads would have filled (the same bytes those loads fill
+  // step's deferred loads would have filled (the same bytes those loads fill
   // once the epilogue is done, so no other wave ever touches them): 32 rows
   // of SRB bytes, 16-byte chunk c of row r at c ^ (r % CH).
   // F32 tiles below 256: K in segments of a.ksteps_split steps (0: one),
   // summed in fp32 registers in order, the rounding of a K split's planes (a
   // segment's MFMA chain is that much shorter).
-  constexpr bool FOLD = F32 && BT < 256;
+  constexpr bool FOLD = F32 && BM < 256;
   txd::f32x4 sum[FOLD ? FN : 1][FOLD ? FM : 1];
   bool folded = false;
   for (int t = 0; t < T; ++t) {
     const TileDesc d = desc(t);
-    const int m0 = d.tm * BT, n0 = d.tn * BT;
+    const int m0 = d.tm * BM, n0 = d.n0;
     // C as a buffer: a store whose row or column block lies past M / N gets
     // an offset past the range and is dropped (N is a multiple of 8, so a
     // 16-byte column block is wholly in or out).  KTAIL: rows of C may have
@@ -596,7 +656,7 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
       for (int k = 1; k < KS - 1; ++k) step(std::false_type{}, VmStep{}, std::false_type{});
     }
     // Scales load just before the last step and are waited for after it
-    // with vmcnt(BLKB), leaving its B loads in flight.  Loads and waits are
+    // with vmcnt(kLastLoads), leaving its own loads in flight.  Loads and waits are
     // written out: the compiler does not count the LDS-DMA loads when it
     // places waits, so its own wait here would be vmcnt(0), a full drain of
     // the next tile's operand loads (vector-memory operations complete in
@@ -642,10 +702,10 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
       load_acc(std::integral_constant<int, 0>{});
       __builtin_amdgcn_sched_barrier(0);
     }
-    const int stage_slot = STG ? sa : sb;  // the slot the last step's A loads go to
+    const int stage_at = op_st == 1 ? sb : STG ? sa : sb;  // where the last step's op_st loads go
     step(std::false_type{}, VmLast{}, std::true_type{});  // the last step (KS >= 2)
     if constexpr (ROWCOL) {
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(BLKB) : "memory");
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kLastLoads) : "memory");
 #pragma unroll
       for (int fm = 0; fm < FM; ++fm) asm volatile("" : "+v"(sav[fm]));
 #pragma unroll
@@ -690,7 +750,7 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
         __builtin_amdgcn_sched_barrier(0);
       });
     }
-    uint8_t *stg = lds + stage_slot * SB + wave * (32 * SRB);
+    uint8_t *stg = lds + stage_at + wave * (32 * SRB);
     // The lane's staging offsets are recomputed for each tile from an opaque
     // copy of the lane index: hoisted out of the tile loop, they would hold
     // registers through the whole K loop (fp8: 238 -> 206 VGPRs).
@@ -699,7 +759,7 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
     const int efrow = el & 15, efg = el >> 4;
     const int srow = el / CH, schunk = el % CH;  // read-back: row SPI i + srow, chunk schunk
     const int n_st = n0 + wn * TN + 8 * schunk;
-    const uint32_t coloff = n_st < a.N ? uint32_t(n_st) * 2u + cmis : kOob;
+    const uint32_t coloff = n_st < d.nend ? uint32_t(n_st) * 2u + cmis : kOob;
     if constexpr (!F32) static_for<FM / 2>([&](auto blk_tag) {
       constexpr int blk = decltype(blk_tag)::value;
       static_for<2>([&](auto u_tag) {
@@ -729,11 +789,16 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
         __builtin_amdgcn_raw_buffer_store_b128(w, crs, voff, 0, 0);
       }
     });
-    // the deferred A s+3 loads (after this wave's last staging reads) and
+    // the deferred loads (after this wave's last staging reads) and
     // the next step's first-half fragments
     __builtin_amdgcn_s_waitcnt((63 & 15) | (7 << 4) | (0 << 8) | ((63 >> 4) << 14));
-    static_for<BLKA>([&](auto j) { load_op(ca, stage_slot, OpA{}, j); });
-    advance(ca, OpA{});
+    if constexpr (op_st == 0) {
+      static_for<BLKA>([&](auto j) { load_op(ca, stage_at, OpA{}, j); });
+      advance(ca, OpA{});
+    } else {
+      static_for<BLKB>([&](auto j) { load_op(cb, stage_at, OpB{}, j); });
+      advance(cb, OpB{});
+    }
     read_start(sa, sb);
   }
   // Drain the trailing (empty-range) loads before the workgroup's LDS is released.

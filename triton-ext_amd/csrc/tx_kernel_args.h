@@ -137,6 +137,11 @@ typedef struct tx_grouped_args {
   int64_t stride_b;
   int64_t stride_sb;
   int64_t stride_bias;  /* fused epilogue (g.epi): bias of problem p at g.bias + p * stride_bias */
+  /* persistent tiles: per m tile {problem, its first row, its rows, m tile
+   * within it}, 16 bytes each, written beside the prefix; NULL: none (the
+   * tile's problem is searched in the prefix) */
+  int32_t *tile_map;
+  int32_t dealt;     /* tile_map holds the groups in the order the prefix kernel deals them */
   int32_t groups;
   int32_t mtiles;       /* m tiles the grid covers */
   int32_t tiles_per;    /* batched: ceil(g.M / 256) */
