@@ -9,6 +9,7 @@
 #include <algorithm>
 #include <climits>
 #include <cstdio>
+#include <cstring>
 
 #include "tx_kernel_args.h"
 #include "tx_ops.h"

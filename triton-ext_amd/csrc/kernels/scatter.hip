@@ -33,6 +33,14 @@ constexpr int kBlock = 1024;
 constexpr int64_t kIter = 4 * kBlock;       // updates per workgroup iteration
 constexpr int kDepth = 3;                   // iterations of loads in flight (pipelined loop)
 constexpr int kDirectSlots = 36864;          // 144 KiB of 4-byte counters
+// fp32 tables in fp64 (see pass64): bins one fp64 table holds, and the bins
+// of a mixed table with its smallest hot range, kHot64 fp64 bins among them.
+constexpr uint32_t kAll64 = kDirectSlots / 2;
+constexpr uint32_t kHot64 = 2048, kMixed = kDirectSlots - kHot64;
+// Updates per workgroup from which a mixed table is considered: with several
+// windows, whose sample is taken anyway, past the fold's chunks; with one,
+// where counting blocks adds 1 to 2 us, from 128 Ki.
+constexpr int kMixedMinChunk = 49152, kMixedMinChunk1 = 131072;        // updates per workgroup
 constexpr int kHashLog2 = 14;                // 16384 slots, 128 KiB keys + values
 constexpr int kHashSlots = 1 << kHashLog2;
 constexpr int kProbes = 4;
@@ -356,17 +364,18 @@ struct Scatter {
   // The best single window for a chunk: counts the first 4 x kBlock updates
   // of the chunk per block of kWinBlock bins, and returns (workgroup-uniform)
   // the start of the `window`-bin window, at a multiple of kWinBlock, that
-  // holds the most of them, with that count and the number sampled.  Every
+  // holds the most of them, with that count, the number sampled and the block
+  // that alone holds the most (`top`: count << 8 | (255 - block)).  Every
   // workgroup of a chunk reads the same sample, so they all agree.  The
   // counts live in `cnt`, the first words of the workgroup's window table
-  // (set up only afterwards).  Needs the whole workgroup; ends with a
-  // barrier.
+  // (set up only afterwards, so the counts stay readable until then).  Needs
+  // the whole workgroup; ends with a barrier.
   static constexpr int kWinBlock = 2048;
   static constexpr int kMaxWinBlocks = 4 * kDirectSlots / kWinBlock;
   static __device__ __forceinline__ void pick_window(const tx_scatter_args &a, int64_t begin, int64_t end, bool vec,
                                      uint32_t window, uint32_t *cnt, uint32_t &base, uint32_t &hits,
-                                     uint32_t &total) {
-    for (int s = threadIdx.x; s < kMaxWinBlocks + 2; s += kBlock) cnt[s] = 0u;
+                                     uint32_t &total, uint32_t &top) {
+    for (int s = threadIdx.x; s < kMaxWinBlocks + 4; s += kBlock) cnt[s] = 0u;
     __syncthreads();
     {
       uint32_t key[4];
@@ -383,10 +392,13 @@ struct Scatter {
       const int nblk = int((uint32_t(a.nbins) + kWinBlock - 1) / kWinBlock);
       const int wblk = int(window / kWinBlock);
       const int ncand = nblk > wblk ? nblk - wblk + 1 : 1;
-      uint32_t sum = 0u, all = 0u;
+      uint32_t sum = 0u, all = 0u, most = 0u;  // most: count << 8 | (255 - block)
       if (lane < ncand)
         for (int i = lane; i < lane + wblk && i < nblk; ++i) sum += cnt[i];
-      for (int i = lane; i < nblk; i += 64) all += cnt[i];
+      for (int i = lane; i < nblk; i += 64) {
+        all += cnt[i];
+        most = max(most, (cnt[i] << 8) | uint32_t(255 - i));
+      }
       // best candidate: most hits, then the lowest start
       uint32_t best = lane < ncand ? (sum << 8) | uint32_t(255 - lane) : 0u;
 #pragma unroll
@@ -394,15 +406,19 @@ struct Scatter {
         const uint32_t o = __shfl_xor(best, off);
         best = o > best ? o : best;
         all += __shfl_xor(all, off);
+        const uint32_t p = __shfl_xor(most, off);
+        most = p > most ? p : most;
       }
       if (lane == 0) {
         cnt[kMaxWinBlocks] = best;
         cnt[kMaxWinBlocks + 1] = all;
+        cnt[kMaxWinBlocks + 2] = most;
       }
     }
     __syncthreads();
     const uint32_t best = __builtin_amdgcn_readfirstlane(cnt[kMaxWinBlocks]);
     total = __builtin_amdgcn_readfirstlane(cnt[kMaxWinBlocks + 1]);
+    top = __builtin_amdgcn_readfirstlane(cnt[kMaxWinBlocks + 2]);
     hits = best >> 8;
     base = uint32_t(255 - (best & 0xFFu)) * kWinBlock;
     __syncthreads();
@@ -410,9 +426,10 @@ struct Scatter {
 
   // Picks the workgroup's hot keys (HotKeys) from the first 4 x kBlock
   // updates of its chunk; on return every lane holds the same set, with
-  // zeroed sums.  Needs the whole workgroup; ends with a barrier.
+  // zeroed sums, and `blocks` (if given) counts the sample per kWinBlock bins.  Needs the whole workgroup; ends with a barrier.
   static __device__ __forceinline__ void sample_hot(const tx_scatter_args &a, uint32_t lo, uint32_t nb, int64_t begin,
-                                    int64_t end, bool vec, uint32_t *aux, HotKeys<OP> &hot) {
+                                    int64_t end, bool vec, uint32_t *aux, HotKeys<OP> &hot,
+                                    uint32_t *blocks = nullptr) {
     uint32_t *skey = aux, *scnt = aux + kSampleSlots;
     for (int s = threadIdx.x; s < kSampleSlots; s += kBlock) {
       skey[s] = kEmpty;
@@ -428,6 +445,7 @@ struct Scatter {
       for (int j = 0; j < 4; ++j) {
         const uint32_t r = key[j] - lo;
         if (!(ok[j] && r < nb)) continue;
+        if (blocks) atomicAdd(&blocks[r / kWinBlock], 1u);
         const uint32_t h = (r * 2654435769u) >> (32 - kSampleLog2);
 #pragma unroll
         for (int p = 0; p < kProbes; ++p) {
@@ -500,10 +518,13 @@ struct Scatter {
   // outside the window go to the bins through the wavefront spill queues in
   // aux; without it they are left to the chunk's other passes.
   static __device__ __forceinline__ void pass(const tx_scatter_args &a, T *table, uint32_t *aux, uint32_t lo, uint32_t nb,
-                              bool spill, int64_t begin, int64_t end, bool vec) {
+                              bool spill, int64_t begin, int64_t end, bool vec, const HotKeys<OP> *sampled = nullptr) {
     for (uint32_t s = threadIdx.x; s < nb; s += kBlock) table[s] = OpTraits<OP>::id();
     HotKeys<OP> hot;
-    if constexpr (OP == FADD) sample_hot(a, lo, nb, begin, end, vec, aux, hot);
+    if constexpr (OP == FADD) {
+      if (sampled) hot = *sampled;
+      else sample_hot(a, lo, nb, begin, end, vec, aux, hot);
+    }
     __syncthreads();
     T *bins = reinterpret_cast<T *>(a.bins);
     uint32_t *q = aux + (threadIdx.x / 64) * 2 * kQueue;
@@ -577,6 +598,151 @@ struct Scatter {
     __syncthreads();  // the table and aux are reused by the next pass
   }
 
+  // fp32 sums in fp64 LDS slots.  ds_add_f64 retires 3 lanes per clock per CU
+  // whatever its addresses (2.6 with every lane on one of 64 bins), where an
+  // fp32 add takes a read and a compare-and-swap (3.5 together, when nothing
+  // is lost), ds_add_f32 (0.33) for the lanes that lose it, and registers for
+  // the hottest keys to keep that rare.  ALL: every bin of the window has an
+  // fp64 slot (nb <= kAll64).  Otherwise the hn bins from window-relative hlo
+  // have, at the start of the table, and the rest of the window keeps fp32
+  // slots behind them (wave_lds_combine; straight ds_add_f32 there was 25 us
+  // slower).  The slots start at -0 like the fp32 table's; an fp64 sum is
+  // rounded to fp32 once, when it is flushed.
+  template <bool ALL, bool SPILL>
+  static __device__ __forceinline__ void apply64(double *t64, float *t32, uint32_t lo, uint32_t nb, uint32_t hlo,
+                                                 uint32_t hn, float *bins, uint32_t nbins, uint32_t *q, uint32_t &qn,
+                                                 SpillRegion &sr, uint32_t key, float x, bool live) {
+    const uint32_t r = key - lo, h = r - hlo;
+    const bool in = r < nb && live;
+    if constexpr (SPILL) spill_push<FADD, float>(q, qn, bins, sr, live && !in && key < nbins, key, x);
+    if constexpr (ALL) {
+      if (in) atomicAdd(&t64[r], double(x));
+    } else {
+      const bool hot = h < hn;
+      if (in && hot) atomicAdd(&t64[h], double(x));
+      wave_lds_combine<FADD, float>(t32, in && !hot, r < hlo ? r : r - hn, x);
+    }
+  }
+
+  template <bool MASK, bool ALL, bool SPILL>
+  static __device__ __forceinline__ void stream64(const tx_scatter_args &a, double *t64, float *t32, uint32_t lo,
+                                                  uint32_t nb, uint32_t hlo, uint32_t hn, uint32_t *q, uint32_t &qn,
+                                                  SpillRegion &sr, int64_t e0, int64_t groups) {
+    float *bins = reinterpret_cast<float *>(a.bins);
+    txd::i32x4 k[kDepth];
+    txd::u32x4 v[kDepth];
+    uint32_t m[kDepth];
+#pragma unroll
+    for (int d = 0; d < kDepth; ++d) fetch<MASK>(a, e0 + d * kIter, k[d], v[d], m[d]);
+    const int64_t last = e0 + (groups * kDepth - 1) * kIter;
+    for (int64_t g = 0; g < groups; ++g) {
+      const int64_t eg = e0 + g * kDepth * kIter;
+#pragma unroll
+      for (int d = 0; d < kDepth; ++d) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          apply64<ALL, SPILL>(t64, t32, lo, nb, hlo, hn, bins, uint32_t(a.nbins), q, qn, sr, uint32_t(k[d][j]),
+                              __uint_as_float(v[d][j]), ((m[d] >> (8 * j)) & 0xFFu) != 0);
+        const int64_t en = eg + (d + kDepth) * kIter;
+        fetch<MASK>(a, en < last ? en : last, k[d], v[d], m[d]);
+      }
+    }
+  }
+
+  template <bool ALL, bool SPILL>
+  static __device__ __forceinline__ void pass64(const tx_scatter_args &a, void *table, uint32_t *aux, uint32_t lo,
+                                                uint32_t nb, uint32_t hlo, uint32_t hn, int64_t begin, int64_t end,
+                                                bool vec) {
+    double *t64 = static_cast<double *>(table);
+    float *t32 = static_cast<float *>(table) + 2 * hn;
+    for (uint32_t s = threadIdx.x; s < hn; s += kBlock) t64[s] = -0.0;
+    if constexpr (!ALL)
+      for (uint32_t s = threadIdx.x; s < nb - hn; s += kBlock) t32[s] = -0.0f;
+    __syncthreads();
+    float *bins = reinterpret_cast<float *>(a.bins);
+    uint32_t *q = aux + (threadIdx.x / 64) * 2 * kQueue;
+    uint32_t qn = 0;
+    SpillRegion sr;
+    if constexpr (SPILL) sr.init(a);
+    int64_t e = begin + 4 * int64_t(threadIdx.x);
+    const int64_t groups = vec ? (end - begin) / (kDepth * kIter) : 0;
+    if (groups > 0) {
+      if (a.mask) stream64<true, ALL, SPILL>(a, t64, t32, lo, nb, hlo, hn, q, qn, sr, e, groups);
+      else stream64<false, ALL, SPILL>(a, t64, t32, lo, nb, hlo, hn, q, qn, sr, e, groups);
+      e += groups * kDepth * kIter;
+    }
+    // remaining iterations: a uniform trip count, lanes past `end` idle
+    const int64_t first = e - 4 * int64_t(threadIdx.x);
+    for (int64_t eb = first; eb < end; eb += kIter) {
+      uint32_t key[4];
+      T val[4];
+      bool ok[4];
+      load4(a, eb + 4 * int64_t(threadIdx.x), end, vec, key, val, ok);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        apply64<ALL, SPILL>(t64, t32, lo, nb, hlo, hn, bins, uint32_t(a.nbins), q, qn, sr, key[j], val[j], ok[j]);
+    }
+    if constexpr (SPILL) {
+      spill_out<FADD, float>(q, qn, bins, sr);
+      sr.close();
+    }
+    __syncthreads();
+    for (uint32_t s = threadIdx.x; s < hn; s += kBlock) {
+      const double v = t64[s];
+      if (__double_as_longlong(v) != __double_as_longlong(-0.0)) atomicAdd(bins + lo + hlo + s, float(v));
+    }
+    if constexpr (!ALL)
+      for (uint32_t s = threadIdx.x; s < nb - hn; s += kBlock) {
+        const float v = t32[s];
+        if (!is_identity<FADD, float>(v)) atomicAdd(bins + lo + (s < hlo ? s : s + hn), v);
+      }
+  }
+
+  // The kMixed-bin window (at a multiple of kWinBlock) that holds block hb and
+  // the most of pick_window's sample, as count << 8 | (255 - first block).
+  // Needs the whole workgroup; ends with a barrier.
+  static __device__ __forceinline__ uint32_t mixed_window(uint32_t nbins, int hb, uint32_t *cnt) {
+    static_assert(int(kHot64) == kWinBlock && kMixed % kWinBlock == 0, "blocks of the sample");
+    if (threadIdx.x < 64) {
+      const int lane = threadIdx.x, wblk = int(kMixed / kWinBlock);
+      const int nblk = int((nbins + kWinBlock - 1) / kWinBlock);
+      const int ncand = nblk > wblk ? nblk - wblk + 1 : 1;  // at most 72 - 17 + 1 = 56
+      uint32_t best = 0u;
+      if (lane < ncand && lane <= hb && hb < lane + wblk) {
+        uint32_t sum = 0u;
+        for (int i = lane; i < lane + wblk && i < nblk; ++i) sum += cnt[i];
+        best = (sum << 8) | uint32_t(255 - lane);
+      }
+#pragma unroll
+      for (int off = 32; off >= 1; off >>= 1) {
+        const uint32_t o = __shfl_xor(best, off);
+        best = o > best ? o : best;
+      }
+      if (lane == 0) cnt[kMaxWinBlocks + 3] = best;
+    }
+    __syncthreads();
+    const uint32_t best = __builtin_amdgcn_readfirstlane(cnt[kMaxWinBlocks + 3]);
+    __syncthreads();
+    return best;
+  }
+
+  // More bins than one window: one pass with the window at `base` when it
+  // holds at least 3/4 of the sample, spilling the rest, else a pass each.
+  static __device__ __forceinline__ void one_or_all(const tx_scatter_args &a, T *table, uint32_t *aux, uint32_t base,
+                                                    uint32_t hits, uint32_t total, int64_t begin, int64_t end,
+                                                    bool vec) {
+    const uint32_t W = uint32_t(a.window), nbins = uint32_t(a.nbins);
+    if (total > 0u && 4u * hits >= 3u * total) {
+      pass(a, table, aux, base, min(W, nbins - base), true, begin, end, vec);
+    } else {
+      for (int w = 0; w < a.splits; ++w)
+        pass(a, table, aux, uint32_t(w) * W, min(W, nbins - uint32_t(w) * W), false, begin, end, vec);
+      SpillRegion sr;  // nothing spilled: every record of the regions unused
+      sr.init(a);
+      sr.close();
+    }
+  }
+
   // Windowed LDS privatisation, one workgroup per chunk of updates.  Up to
   // `window` bins the table holds them all and one pass does the chunk.
   // Beyond that the bin range is cut into `splits` windows of `window` bins
@@ -586,7 +752,7 @@ struct Scatter {
   // of the chunk); otherwise it makes one pass per window, each reading the
   // whole chunk.
   static __device__ __forceinline__ void windowed(const tx_scatter_args &a) {
-    __shared__ T table[kDirectSlots];
+    __shared__ __attribute__((aligned(16))) T table[kDirectSlots];
     __shared__ uint32_t aux[kAuxWords];
     const int64_t begin = int64_t(blockIdx.x) * a.per_block;
     if (begin >= a.n) return;  // uniform: the whole workgroup leaves
@@ -594,18 +760,60 @@ struct Scatter {
     const bool vec = ((reinterpret_cast<uintptr_t>(a.idx) | reinterpret_cast<uintptr_t>(a.val)) & 15) == 0 &&
                      (!a.mask || (reinterpret_cast<uintptr_t>(a.mask) & 3) == 0);
     const uint32_t W = uint32_t(a.window), nbins = uint32_t(a.nbins);
-    if (a.splits > 1) {
-      uint32_t base, hits, total;
-      pick_window(a, begin, end, vec, W, reinterpret_cast<uint32_t *>(table), base, hits, total);
-      if (total > 0u && 4u * hits >= 3u * total) {
-        pass(a, table, aux, base, min(W, nbins - base), true, begin, end, vec);
-      } else {
-        for (int w = 0; w < a.splits; ++w)
-          pass(a, table, aux, uint32_t(w) * W, min(W, nbins - uint32_t(w) * W), false, begin, end, vec);
-        SpillRegion sr;  // nothing spilled: every record of the regions unused
-        sr.init(a);
-        sr.close();
+    if constexpr (OP == FADD) {
+      // fp64 slots for all bins; or, past the fold's chunks, for the block of
+      // bins that draws at least half of a sample, when the window spills at
+      // most a quarter (elsewhere lanes would often split between the two
+      // kinds of slot: 20,000 flat bins 101 -> 112 us).
+      // 64 Mi Zipf(1.1) updates, fp32 -> fp64 slots (same box): 256 bins 168 ->
+      // 102 us (flat keys 323 -> 82), 4096 147 -> 95, 18,000 152 -> 103;
+      // mixed, 30,000 bins 160 -> 149, 65,536 194 -> 178.  1 Mi into 1000 bins 30
+      // -> 13 us (no hot-key sample), 64 Ki into 300 35 -> 13.
+      if (nbins <= kAll64) {
+        pass64<true, false>(a, table, aux, 0u, nbins, 0u, nbins, begin, end, vec);
+        return;
       }
+      if (a.splits == 1 && nbins <= kMixed && a.per_block >= kMixedMinChunk1) {
+        // all bins in the window, as many hot ones as fit beside the rest
+        uint32_t *cnt = reinterpret_cast<uint32_t *>(table);
+        const int nblk = int((nbins + kWinBlock - 1) / kWinBlock);
+        for (int i = threadIdx.x; i < nblk; i += kBlock) cnt[i] = 0u;
+        HotKeys<OP> hot;
+        sample_hot(a, 0u, nbins, begin, end, vec, aux, hot, cnt);  // (its first barrier covers the zeros)
+        uint32_t total = 0u, top = 0u, at = 0u;
+        for (int i = 0; i < nblk; ++i) {
+          const uint32_t c = __builtin_amdgcn_readfirstlane(cnt[i]);
+          total += c;
+          if (c > top) top = c, at = uint32_t(i);
+        }
+        __syncthreads();
+        if (total > 0u && 2u * top >= total) {
+          const uint32_t hn = (kDirectSlots - nbins) / kWinBlock * kWinBlock;  // < nbins
+          const uint32_t hlo = min(at * kWinBlock, nbins - hn);
+          pass64<false, false>(a, table, aux, 0u, nbins, hlo, hn, begin, end, vec);
+        } else {
+          pass(a, table, aux, 0u, nbins, false, begin, end, vec, &hot);
+        }
+        return;
+      }
+    }
+    if (a.splits > 1) {
+      uint32_t base, hits, total, top;
+      uint32_t *cnt = reinterpret_cast<uint32_t *>(table);
+      pick_window(a, begin, end, vec, W, cnt, base, hits, total, top);
+      if constexpr (OP == FADD) {
+        if (a.per_block >= kMixedMinChunk && total > 0u && 2u * (top >> 8) >= total) {
+          const int hb = 255 - int(top & 0xFFu);
+          const uint32_t m = mixed_window(nbins, hb, cnt);
+          if (4u * (m >> 8) >= 3u * total) {
+            const uint32_t at = uint32_t(255 - (m & 0xFFu)) * kWinBlock, nb = min(kMixed, nbins - at);
+            const uint32_t hlo = uint32_t(hb) * kWinBlock - at;
+            pass64<false, true>(a, table, aux, at, nb, hlo, min(kHot64, nb - hlo), begin, end, vec);
+            return;
+          }
+        }
+      }
+      one_or_all(a, table, aux, base, hits, total, begin, end, vec);
       return;
     }
     pass(a, table, aux, 0u, min(W, nbins), false, begin, end, vec);
@@ -647,7 +855,7 @@ struct Scatter {
             uint32_t k = __atomic_load_n(&keys[slot], __ATOMIC_RELAXED);
             if (k == kEmpty) k = atomicCAS(&keys[slot], kEmpty, key[j]);
             if (k == kEmpty || k == key[j]) {
-              atomic_combine<OP, T>(&vals[slot], val[j]);
+              wave_lds_combine<OP, T>(vals, true, slot, val[j]);
               spill = false;
               break;
             }
