@@ -546,8 +546,8 @@ struct Epilogue {
   bool on() const { return bias || act != EPI_ACT_NONE || out_kind != EPI_OUT_BF16; }
 };
 
-// Skinny and generic kernels write scaled fp32 sums to a.part (stream
-// scratch slot 1) when an epilogue is requested; this pass finishes them.
+// Generic kernels write scaled fp32 sums to a.part (stream scratch slot 1)
+// when an epilogue is requested; this pass finishes them.
 tx_status epilogue_pass(tx_gemm_args &args, hipStream_t s) {
   hipFunction_t fn;
   TX_TRY(get_kernel(CodeObject::GemmFp8, "tx_gemm_fp8_epilogue", &fn));
@@ -580,7 +580,7 @@ static tx_status dot_fp8_impl(const char *what, const void *A, tx_dtype a_type, 
     args.out_mul = epi.out_mul;
     args.epi = 1;
   }
-  // skinny / generic kernels with an epilogue: scaled sums into scratch first
+  // generic kernels with an epilogue: scaled sums into scratch first
   ScratchLease sums;
   auto with_sums = [&]() -> tx_status {
     TX_TRY(sums.acquire(s, 1, size_t(M) * size_t(N) * sizeof(float)));
@@ -600,9 +600,7 @@ static tx_status dot_fp8_impl(const char *what, const void *A, tx_dtype a_type, 
     std::snprintf(kname, sizeof kname, "tx_gemm_fp8_%s_%s_skinny_w%d_m%d", fa, fb, waves, mb);
     hipFunction_t fn;
     TX_TRY(get_kernel(CodeObject::GemmFp8, kname, &fn));
-    if (with_epi) TX_TRY(with_sums());
-    TX_TRY(launch(fn, unsigned(grid), 1, unsigned(64 * waves), s, &args, sizeof args, kname));
-    return with_epi ? epilogue_pass(args, s) : TX_SUCCESS;
+    return launch(fn, unsigned(grid), 1, unsigned(64 * waves), s, &args, sizeof args, kname);
   }
   std::snprintf(kname, sizeof kname, "tx_gemm_fp8_%s_%s_fast%s", fa, fb, with_epi ? "_epi" : "");
   if (fast_ok(A, lda, B, ldb, K, M, N))

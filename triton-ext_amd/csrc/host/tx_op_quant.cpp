@@ -82,13 +82,19 @@ tx_status quantize_rowwise(const void *x, tx_dtype x_type, int64_t ldx, void *q,
   if (rows == 0 || K == 0) return TX_SUCCESS;
   if (!aligned(scales, 4)) return fail(TX_INVALID_ARGUMENT, "%s: scales not 4-byte aligned", what);
   char kname[64];
-  std::snprintf(kname, sizeof kname, "tx_quant_row_%s_%s", q_name(q_type), x_name(x_type));
+  const int64_t ve = x_type == TX_F32 ? 4 : 8;  // elements per 16-byte vector
+  tx_quant_args a{x, static_cast<uint8_t *>(q), scales, ldx, ldq, 0, rows, K,
+                  quant_vec(x, x_type, ldx, q, ldq, K, int(ve)) ? 1 : 0, 0};
+  // 1024 threads per row (kWideRow in fp8_codec.hip): rows of more vectors
+  // than 256 threads keep in registers (K > 8192), and rows of at least two
+  // per thread when there are fewer than two such workgroups per CU
+  const bool wide = a.vec && K % ve == 0 && K <= 16384 &&
+                    (K > 8192 || (K / ve > 256 && rows < 2 * int64_t(cu_count())));
+  std::snprintf(kname, sizeof kname, "tx_quant_row_%s%s_%s", wide ? "wide_" : "", q_name(q_type), x_name(x_type));
   hipFunction_t fn;
   TX_TRY(get_kernel(CodeObject::Fp8Codec, kname, &fn));
-  tx_quant_args a{x, static_cast<uint8_t *>(q), scales, ldx, ldq, 0, rows, K,
-                  quant_vec(x, x_type, ldx, q, ldq, K, x_type == TX_F32 ? 4 : 8) ? 1 : 0, 0};
   const int64_t grid = std::min<int64_t>(rows, int64_t(cu_count()) * 16);
-  return launch(fn, unsigned(grid), 1, 256, static_cast<hipStream_t>(stream), &a, sizeof a, kname);
+  return launch(fn, unsigned(grid), 1, wide ? 1024 : 256, static_cast<hipStream_t>(stream), &a, sizeof a, kname);
 }
 
 // tx.quantize_mx: {q (result), scales (result), x, rows, K, ldx, ldq, ld_scales, x_type, q_type}

@@ -667,13 +667,14 @@ __device__ __forceinline__ float vec_absmax(const txd::u32x4 &p, float amax) {
 }
 
 // Workgroup-wide absmax (NaN never enters: absmax_step drops it).
+template <int NB = kBlock>
 __device__ __forceinline__ float block_absmax(float amax, float *red) {
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) amax = absmax_step(amax, __shfl_xor(amax, o));
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = amax;
   __syncthreads();
 #pragma unroll
-  for (int w = 0; w < kBlock / 64; ++w) amax = absmax_step(amax, red[w]);
+  for (int w = 0; w < NB / 64; ++w) amax = absmax_step(amax, red[w]);
   __syncthreads();  // red is reused by the next row
   return amax;
 }
@@ -692,15 +693,24 @@ constexpr int RowRegs = XT == 0 ? 8 : 4;
 // (fp32 throughout; NaN inputs stay NaN).  One workgroup per row; fp32 rows
 // that fit are read once into registers, other rows take a pass for amax
 // and a second pass (from cache) for the codes.
-template <int FMT, int XT>
+// Wide variant, 1024 threads per row of up to 2 (bf16) or 4 (fp32) vectors
+// each (K <= 16384): rows too long for the registers above, which were read
+// twice, and few rows, whose 256-thread workgroups leave the chip idle.
+// bf16 512 x 14336 8.8 -> 7.7 us, 4096 x 14336 45 -> 42, 8192 x 16384 103 ->
+// 84; fp32 4096 x 14336 88 -> 62, 8192 x 16384 184 -> 130.
+constexpr int kWideRow = 1024;
+template <int XT>
+constexpr int kWideRegs = XT == 0 ? 4 : 2;
+
+template <int FMT, int XT, int NB = kBlock>
 __device__ __forceinline__ void quant_row(const tx_quant_args &a) {
   constexpr float FMAX = FMT == E4M3FN ? 448.0f : 57344.0f;
   constexpr int VE = XT == 0 ? 4 : 8;  // elements per 16-byte load
-  __shared__ float red[kBlock / 64];
+  __shared__ float red[NB / 64];
   float *scales = static_cast<float *>(a.scales);
   const int tid = threadIdx.x;
-  constexpr int RR = RowRegs<XT>;
-  const bool in_regs = a.vec && a.K % VE == 0 && a.K / VE <= int64_t(kBlock) * RR;
+  constexpr int RR = NB == kBlock ? RowRegs<XT> : kWideRegs<XT>;
+  const bool in_regs = a.vec && a.K % VE == 0 && a.K / VE <= int64_t(NB) * RR;
   if (in_regs) {
     const int nvec = int(a.K / VE);
     for (int64_t r = blockIdx.x; r < a.rows; r += gridDim.x) {
@@ -708,21 +718,21 @@ __device__ __forceinline__ void quant_row(const tx_quant_args &a) {
       txd::u32x4 p[RR];
 #pragma unroll
       for (int j = 0; j < RR; ++j) {
-        const int i = tid + kBlock * j;
+        const int i = tid + NB * j;
         if (i < nvec) p[j] = *reinterpret_cast<const txd::u32x4 *>(xrow + 16 * int64_t(i));
       }
       float amax = 0.0f;
 #pragma unroll
       for (int j = 0; j < RR; ++j)
-        if (tid + kBlock * j < nvec) amax = vec_absmax<XT>(p[j], amax);
-      amax = block_absmax(amax, red);
+        if (tid + NB * j < nvec) amax = vec_absmax<XT>(p[j], amax);
+      amax = block_absmax<NB>(amax, red);
       if (amax == 0.0f) amax = 1.0f;
       const float mult = FMAX / amax;
       if (tid == 0) scales[r] = amax / FMAX;
       uint8_t *qrow = a.q + r * a.ldq;
 #pragma unroll
       for (int j = 0; j < RR; ++j) {
-        const int i = tid + kBlock * j;
+        const int i = tid + NB * j;
         if (i < nvec) row_codes<FMT, XT>(p[j], mult, qrow, i);
       }
     }
@@ -733,16 +743,16 @@ __device__ __forceinline__ void quant_row(const tx_quant_args &a) {
     uint8_t *qrow = a.q + r * a.ldq;
     const int64_t nvec = a.vec ? a.K / VE : 0;
     float amax = 0.0f;
-    for (int64_t i = tid; i < nvec; i += kBlock)
+    for (int64_t i = tid; i < nvec; i += NB)
       amax = vec_absmax<XT>(*reinterpret_cast<const txd::u32x4 *>(xrow + 16 * i), amax);
-    for (int64_t i = nvec * VE + tid; i < a.K; i += kBlock) amax = absmax_step(amax, load_x<XT>(xrow, i));
-    amax = block_absmax(amax, red);
+    for (int64_t i = nvec * VE + tid; i < a.K; i += NB) amax = absmax_step(amax, load_x<XT>(xrow, i));
+    amax = block_absmax<NB>(amax, red);
     if (amax == 0.0f) amax = 1.0f;
     const float mult = FMAX / amax;
     if (tid == 0) scales[r] = amax / FMAX;
-    for (int64_t i = tid; i < nvec; i += kBlock)
+    for (int64_t i = tid; i < nvec; i += NB)
       row_codes<FMT, XT>(*reinterpret_cast<const txd::u32x4 *>(xrow + 16 * i), mult, qrow, i);
-    for (int64_t i = nvec * VE + tid; i < a.K; i += kBlock)
+    for (int64_t i = nvec * VE + tid; i < a.K; i += NB)
       qrow[i] = uint8_t(encode_rtne<FMT, false>(__float_as_uint(clamp_keep_nan<FMT>(load_x<XT>(xrow, i) * mult))));
   }
 }
@@ -756,6 +766,9 @@ __device__ __forceinline__ void quant_row(const tx_quant_args &a) {
   }                                                                                         \
   TX_KERNEL void __launch_bounds__(kBlock) tx_quant_row_##FN##_##XN(const tx_quant_args a) { \
     quant_row<FMT, XT>(a);                                                                  \
+  }                                                                                         \
+  TX_KERNEL void __launch_bounds__(kWideRow) tx_quant_row_wide_##FN##_##XN(const tx_quant_args a) { \
+    quant_row<FMT, XT, kWideRow>(a);                                                        \
   }
 
 TX_QUANT_KERNELS(e4m3fn, E4M3FN, f32, 0)

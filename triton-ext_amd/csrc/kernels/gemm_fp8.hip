@@ -104,7 +104,7 @@ TX_GEMM_FP8_SKINNY_ALL(e5m2, e4m3fn, EL_E5M2, EL_E4M3)
 
 TX_KERNEL void __launch_bounds__(256) tx_gemm_fp8_pad_rows(const tx_pad_args a) { pad_rows<1>(a); }
 
-// Epilogue pass of the skinny and generic kernels: their scaled fp32 sums
+// Epilogue pass of the generic kernels: their scaled fp32 sums
 // (a.part, M x N) through bias, activation and the output conversion into C.
 TX_KERNEL void __launch_bounds__(256) tx_gemm_fp8_epilogue(const tx_gemm_args a) {
   const int64_t total = int64_t(a.M) * a.N;
