@@ -70,12 +70,19 @@ def get_fp8_format_name(dtype) -> str:
         f"get_fp8_format_name only supports float8_e5m2 (e5m2) and float8_e4m3fn (e4m3), got {dtype}")
 
 
-def _stream(t: torch.Tensor):
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+# The current stream's handle without building a torch.cuda.Stream object (2.0 us
+# of a call's 11 on the host; 0.1 this way): what torch's own generated code calls.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
+def _stream(t: torch.Tensor) -> int:
+    if _raw_stream is None:
+        return torch.cuda.current_stream(t.device).cuda_stream
+    return _raw_stream(t.get_device())
 
 
 def _ptr(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 def _on_gpu(*ts):
