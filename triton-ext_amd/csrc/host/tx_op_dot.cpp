@@ -121,15 +121,15 @@ constexpr int64_t kStripKernelCols = 8, kStripKernelRows = 4;
 
 // The persistent 4-wavefront kernel (gemm_persist.h) takes the 256 x 256
 // products it was built for: no fused epilogue or K split, at least two
-// 128-byte K steps, N a multiple of 8, C addressable with 32-bit byte
-// offsets.  `base`_persist: K a whole number of steps, C rows 16-byte
-// aligned; `base`_persist_kt (16-bit operands, es == 2): any K and any C
+// 128-byte K steps, C addressable with 32-bit byte offsets.  `base`_persist: K
+// a whole number of steps, N a multiple of 8, C rows 16-byte aligned;
+// `base`_persist_kt (16-bit operands, es == 2): any K, any N and any C
 // alignment.  Returns the kernel suffix, or nullptr.
 const char *persist_variant(const tx_gemm_args &args, int64_t k_bytes, int es) {
-  if (args.epi || args.splits > 1 || k_bytes < 256 || args.N % 8 != 0) return nullptr;
+  if (args.epi || args.splits > 1 || k_bytes < 256) return nullptr;
   const int64_t c_bytes = ((int64_t(args.M) - 1) * args.ldc + args.N) * 2;
   if (c_bytes + 16 >= (int64_t(1) << 31)) return nullptr;
-  if (k_bytes % 128 == 0 && aligned(args.C, 16) && args.ldc % 8 == 0) return "_persist";
+  if (k_bytes % 128 == 0 && args.N % 8 == 0 && aligned(args.C, 16) && args.ldc % 8 == 0) return "_persist";
   return es == 2 && aligned(args.C, 2) ? "_persist_kt" : nullptr;
 }
 
@@ -210,8 +210,14 @@ tx_status launch_fast(const char *base, const char *reduce, CodeObject co, tx_ge
     // small_persist_tile picks (16-bit operands), no K split
     const char *pv = persist_variant(args, k_bytes, es);
     const int bt = small_persist_tile(args.M, args.N, k_bytes, cus);
-    if (bt && pv && std::strcmp(pv, "_persist") == 0) {
-      std::snprintf(kname, sizeof kname, "%s_persist%d", base, bt);
+    // (ragged operands: not where a nearly empty last round would cost more
+    // than half of the rest: 2048 x 2050 x 2048, 272 tiles, 33 us here, 30 us in
+    // 256 x 128 tiles; 999 x 2001 x 1024, 512 tiles of 64 x 64, 43 us there, 13
+    // here; 4000 x 1001 x 500, 51 there, 12 here)
+    const int64_t tiles = bt ? ((args.M + bt - 1) / bt) * ((args.N + bt - 1) / bt) : 0;
+    const bool even = 2 * ((tiles + cus - 1) / cus) * cus <= 3 * tiles || tiles <= cus;
+    if (bt && pv && (even || std::strcmp(pv, "_persist") == 0)) {
+      std::snprintf(kname, sizeof kname, "%s_persist%d%s", base, bt, pv + std::strlen("_persist"));
       args.tiles_m = int32_t((args.M + bt - 1) / bt);
       args.tiles_n = int32_t((args.N + bt - 1) / bt);
       args.group_m = std::min<int32_t>(kGroupM, args.tiles_m);
@@ -258,6 +264,9 @@ tx_status launch_fast(const char *base, const char *reduce, CodeObject co, tx_ge
 // Returns TX_UNSUPPORTED without launching anything when that is not
 // possible, and the caller takes the generic kernel.
 constexpr int64_t kPadMinWork = int64_t(1) << 30;
+// (16-bit operands, whose copies then take the small persistent tiles: 333 x
+// 777 x 555 45 us on the generic tile, 15 us with the copies; 411^3 37 -> 15.)
+constexpr int64_t kPadMinWork16 = int64_t(1) << 26;
 
 // Widest source load (8, 4, 2 or 1 bytes) that divides the base address,
 // the row pitch and the row length of a padded copy's source.
@@ -304,7 +313,7 @@ tx_status pad_operands(const char *pad, CodeObject co, tx_gemm_args &args, int e
 
 tx_status launch_padded(const char *base, const char *reduce, const char *pad, CodeObject co,
                         tx_gemm_args &args, int es, hipStream_t s) {
-  if (int64_t(args.M) * args.N * args.K < kPadMinWork) return TX_UNSUPPORTED;
+  if (int64_t(args.M) * args.N * args.K < (es == 2 ? kPadMinWork16 : kPadMinWork)) return TX_UNSUPPORTED;
   ScratchLease ws;  // held until every launch using it is enqueued
   TX_TRY(pad_operands(pad, co, args, es, s, ws));
   return launch_fast(base, reduce, co, args, int64_t(args.K) * es, es, s, true);

@@ -56,8 +56,8 @@ TX_GEMM16_FAST(f16, EL_F16, _out_bf16, OUT_BF16)
 // The persistent 4-wavefront tile (one workgroup per CU; see gemm_persist.h)
 // for products of at least one 256 x 256 tile per CU whose K is a whole
 // number (>= 2) of 64-element steps, N a multiple of 8 and C 16-byte aligned;
-// _persist_kt: any K of at least 128 elements, rows of A and B 4-byte
-// aligned, C rows of any alignment; _persist_kn: B row-major K x N (ldb
+// _persist[128|64]_kt: any K of at least 128 elements, rows of A and B 4-byte
+// aligned, any N, C rows of any alignment; _persist_kn: B row-major K x N (ldb
 // elements per K row), K a whole number of 64-element steps, B and its rows
 // 16-byte aligned; _persist128[_kn] / _persist64[_kn]: the same on 128 x 128
 // / 64 x 64 tiles, for products with fewer 256 x 256 / 128 x 128 tiles than
@@ -86,11 +86,22 @@ TX_GEMM16_FAST(f16, EL_F16, _out_bf16, OUT_BF16)
   TX_KERNEL void __launch_bounds__(256) tx_gemm_##PFX##_fast##SFX##_persist64_kn(const tx_gemm_args a) { \
     gemm_persist<GemmCfg<EL, EL, 256, 256, 2, 2, 16>, OUT, false, false, true, 64>(a);                     \
   }
+#define TX_GEMM16_PERSIST_KT(PFX, EL, SFX, OUT)                                                           \
+  TX_KERNEL void __launch_bounds__(256) tx_gemm_##PFX##_fast##SFX##_persist128_kt(const tx_gemm_args a) { \
+    gemm_persist<GemmCfg<EL, EL, 256, 256, 2, 2, 16>, OUT, false, true, false, 128>(a);                    \
+  }                                                                                                       \
+  TX_KERNEL void __launch_bounds__(256) tx_gemm_##PFX##_fast##SFX##_persist64_kt(const tx_gemm_args a) {  \
+    gemm_persist<GemmCfg<EL, EL, 256, 256, 2, 2, 16>, OUT, false, true, false, 64>(a);                     \
+  }
 
 TX_GEMM16_PERSIST(bf16, EL_BF16, , OUT_BF16)
 TX_GEMM16_PERSIST(bf16, EL_BF16, _out_f16, OUT_F16)
 TX_GEMM16_PERSIST(f16, EL_F16, , OUT_F16)
 TX_GEMM16_PERSIST(f16, EL_F16, _out_bf16, OUT_BF16)
+TX_GEMM16_PERSIST_KT(bf16, EL_BF16, , OUT_BF16)
+TX_GEMM16_PERSIST_KT(bf16, EL_BF16, _out_f16, OUT_F16)
+TX_GEMM16_PERSIST_KT(f16, EL_F16, , OUT_F16)
+TX_GEMM16_PERSIST_KT(f16, EL_F16, _out_bf16, OUT_BF16)
 
 // tt.dot with its accumulator operand, D = A.B + C in fp32 (a.acc, NULL: no
 // C), on the persistent tiles: tx_gemm_{bf16,f16}_fast_acc_persist...  The

@@ -759,7 +759,11 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
     const int efrow = el & 15, efg = el >> 4;
     const int srow = el / CH, schunk = el % CH;  // read-back: row SPI i + srow, chunk schunk
     const int n_st = n0 + wn * TN + 8 * schunk;
-    const uint32_t coloff = n_st < d.nend ? uint32_t(n_st) * 2u + cmis : kOob;
+    // KTAIL: N may be any; the lanes whose 8 columns straddle it (in a last
+    // column tile) store them one by one.
+    const bool straddle = KTAIL && (d.nend & 7) != 0 && n0 + BN > d.nend;
+    const int cols = KTAIL ? d.nend - n_st : 8;  // valid columns from n_st on
+    const uint32_t coloff = n_st < d.nend && (!KTAIL || cols >= 8) ? uint32_t(n_st) * 2u + cmis : kOob;
     if constexpr (!F32) static_for<FM / 2>([&](auto blk_tag) {
       constexpr int blk = decltype(blk_tag)::value;
       static_for<2>([&](auto u_tag) {
@@ -787,6 +791,14 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
         const int m = m0 + wm * TM + blk * 32 + r;
         const uint32_t voff = (m >= d.rows || coloff == kOob) ? kOob : uint32_t(m) * uint32_t(a.ldc) * 2u + coloff;
         __builtin_amdgcn_raw_buffer_store_b128(w, crs, voff, 0, 0);
+        if (straddle && cols > 0 && cols < 8 && m < d.rows) {
+#pragma unroll
+          for (int t = 0; t < 7; ++t)
+            if (t < cols)
+              __builtin_amdgcn_raw_buffer_store_b16(uint16_t(w[t / 2] >> (16 * (t & 1))), crs,
+                                                    uint32_t(m) * uint32_t(a.ldc) * 2u + uint32_t(n_st + t) * 2u + cmis,
+                                                    0, 0);
+        }
       }
     });
     // the deferred loads (after this wave's last staging reads) and
