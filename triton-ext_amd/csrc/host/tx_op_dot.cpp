@@ -145,6 +145,25 @@ int small_persist_tile(int64_t M, int64_t N, int64_t k_bytes, int64_t cus) {
   return (k_bytes + 127) / 128 <= kSmallMaxSteps ? 64 : 0;
 }
 
+// fp8 products with fewer 256 x 256 tiles than CUs: whether the 128 x 128
+// persistent tile beats the 256 x 128 one with its K split and reduce, from
+// what they measured: a K step of a round 0.5 us (32 KiB a CU, the rate its
+// LDS loads arrive at) against 1.0 us (48 KiB), and for a K split its planes
+// (8 bytes per split and element at 5 TB/s) and 4 us of a second launch.
+// Before -> here: 2048^3 29.2 -> 13.2 us, 1024 x 4096 x 4096 31.4 -> 20.9, 512 x
+// 8192 x 2048 25.5 -> 12.7, 700 x 2048 x 2048 22.6 -> 10.6, 1500 x 6000 x 3072 41.2
+// -> 38.7; left to the other tile: 512 x 14336 x 4096, 1024 x 1024 x 8192.
+bool fp8_persist128(int64_t M, int64_t N, int64_t ksteps, int64_t cus) {
+  const int64_t t128 = ((M + 127) / 128) * ((N + 127) / 128), tn = ((M + 255) / 256) * ((N + 127) / 128);
+  int64_t splits = std::max<int64_t>(1, std::min({kMaxSplits, cus / tn, ksteps / kMinStepsPerSplit}));
+  const int64_t per = (ksteps + splits - 1) / splits;
+  splits = (ksteps + per - 1) / per;
+  const double here = double((t128 + cus - 1) / cus) * double(ksteps) * 0.5;
+  const double there = double((tn * splits + cus - 1) / cus) * double(per) +
+                       (splits > 1 ? 4.0 + double(splits) * double(M) * double(N) * 8.0 / 5e6 : 0.0);
+  return here < 0.9 * there;
+}
+
 // `narrow` sends the whole product to the 256 x 128 tile (the column tail
 // of a wide product: at most kStripMaxN columns, and any K the 256 x 128
 // tile takes, decided before the main part is launched).
@@ -204,6 +223,21 @@ tx_status launch_fast(const char *base, const char *reduce, CodeObject co, tx_ge
       return launch_fast(base, reduce, co, strip_args, k_bytes, es, s, persist, true);
     }
     return launch_big(args);
+  }
+  if (!narrow && persist && es == 1) {
+    // (the fused epilogue stores by itself, to C of any alignment)
+    const bool ok = args.epi ? args.splits <= 1 && k_bytes >= 256 && k_bytes % 128 == 0 && args.N % 8 == 0
+                             : persist_variant(args, k_bytes, es) != nullptr;
+    if (ok && fp8_persist128(args.M, args.N, k_bytes / 128, cus)) {
+      std::snprintf(kname, sizeof kname, "%s_persist128", base);
+      args.tiles_m = int32_t((args.M + 127) / 128);
+      args.tiles_n = int32_t((args.N + 127) / 128);
+      args.group_m = std::min<int32_t>(kGroupM, args.tiles_m);
+      hipFunction_t fn;
+      TX_TRY(get_kernel(co, kname, &fn));
+      const int64_t grid = std::min<int64_t>(int64_t(args.tiles_m) * args.tiles_n, cus);
+      return launch(fn, unsigned(grid), 1, 64 * kPersistWaves, s, &args, sizeof args, kname);
+    }
   }
   if (!narrow && persist && es == 2) {
     // fewer 256 x 256 tiles than CUs: the persistent tile at the edge

@@ -46,12 +46,20 @@ TX_GEMM_FP8_FAST(e5m2, e4m3fn, EL_E5M2, EL_E4M3)
 
 // The persistent 4-wavefront tile (one workgroup per CU; see gemm_persist.h)
 // for products of at least one 256 x 256 tile per CU whose K is a whole
-// number (>= 2) of 128-byte steps, N a multiple of 8 and C 16-byte aligned.
+// number (>= 2) of 128-byte steps, N a multiple of 8 and C 16-byte aligned;
+// _persist128: on 128 x 128 tiles, for products with fewer (fp8_persist128 in
+// tx_op_dot.cpp).
 #include "gemm_persist.h"
 
 #define TX_GEMM_FP8_PERSIST(FA, FB, ELA, ELB)                                                               \
   TX_KERNEL void __launch_bounds__(256) tx_gemm_fp8_##FA##_##FB##_fast_persist(const tx_gemm_args a) {    \
     gemm_persist<GemmCfg<ELA, ELB, 256, 256, 2, 2, 16>>(a);                                                  \
+  }                                                                                                         \
+  TX_KERNEL void __launch_bounds__(256) tx_gemm_fp8_##FA##_##FB##_fast_persist128(const tx_gemm_args a) { \
+    gemm_persist<GemmCfg<ELA, ELB, 256, 256, 2, 2, 16>, OUT_BF16, false, false, false, 128>(a);              \
+  }                                                                                                         \
+  TX_KERNEL void __launch_bounds__(256) tx_gemm_fp8_##FA##_##FB##_fast_epi_persist128(const tx_gemm_args a) { \
+    gemm_persist<GemmCfg<ELA, ELB, 256, 256, 2, 2, 16>, OUT_BF16, false, false, false, 128, 128, true>(a);   \
   }                                                                                                         \
   TX_KERNEL void __launch_bounds__(256) tx_gemm_fp8_##FA##_##FB##_grouped_persist(const tx_grouped_args q) { \
     gemm_persist<GemmCfg<ELA, ELB, 256, 256, 2, 2, 16>, OUT_BF16, true>(q.g, &q);                            \

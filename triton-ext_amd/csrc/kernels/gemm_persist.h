@@ -54,7 +54,7 @@
 // resource for C (stores past M / N are dropped).  OUT_F32 (tt.dot with its
 // accumulator operand): D = A.B + C in fp32 is written straight from the
 // accumulators, C's loads for the first row blocks issued before the last K
-// step.  The first K step of each
+// step.  EPI: the fp8 dot's fused epilogue, likewise from the accumulators.  The first K step of each
 // tile starts its MFMAs from a zero accumulator operand, so the accumulators
 // are never cleared explicitly.
 #pragma once
@@ -144,11 +144,12 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rsrc(const void *base, in
 // 4 chunks on 16 of 256 bytes (for 128-byte rows, two to 256 bytes of
 // banks: on 8 of 128 and on 16 half-row positions).
 template <class C, int OUT = OUT_BF16, bool GROUPED = false, bool KTAIL = false, bool BKN = false, int BM = 256,
-          int BN = BM>
+          int BN = BM, bool EPI = false>
 __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_grouped_args *q = nullptr) {
   using namespace fast;
   static_assert(OUT == OUT_BF16 || (OUT == OUT_F16 && !C::FP8) || (OUT == OUT_F32 && !C::FP8),
                 "bf16 output, or fp16 / fp32 (+ accumulator) out of 16-bit operands");
+  static_assert(!EPI || (C::FP8 && !GROUPED && BM == 128 && BN == 128), "fused epilogue: fp8, 128 x 128");
   constexpr bool F32 = OUT == OUT_F32;
   static_assert(!KTAIL || (!C::FP8 && !GROUPED), "ragged K: 16-bit operands, one product");
   static_assert(!BKN || (!C::FP8 && !GROUPED && !KTAIL), "row-major B: 16-bit operands, whole K steps");
@@ -158,7 +159,7 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
   constexpr int TM = BM / 2, TN = BN / 2, FM = TM / 16, FN = TN / 16;
   // MFMAs of a K step's half (16-bit: K half h; fp8: half of the columns)
   constexpr int NM = C::FP8 ? FM * FN / 2 : FM * FN, NF = FM + FN, NR = NF;
-  static_assert(!C::FP8 || BN == 256, "fp8: 256 columns");
+  static_assert(!C::FP8 || BN >= 128, "fp8: at least 128 columns");
   constexpr int SBA = BM * kStep, SBB = BN * kStep;  // one operand of one K step
   constexpr int BLKA = SBA / 1024 / NW, BLKB = SBB / 1024 / NW, ND = BLKA + BLKB;
   constexpr int RW = NM >= 2 ? NM / 2 : 1;
@@ -566,8 +567,9 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
         constexpr int g = i / HF, j = i % HF;
         if constexpr (j == HF - 1) read_piece(na, nb, std::integral_constant<int, g>{}, H0{});
         if constexpr (j == 0 && g > 0) read_piece(na, nb, std::integral_constant<int, g - 1>{}, H1{});
-        if constexpr (j == 1 && g < 4)
-          read_piece(na, nb, std::integral_constant<int, FM + g / 2>{}, std::integral_constant<int, g % 2>{});
+        constexpr int p = HF == 4 ? (j == 1 ? g : 4) : i;  // piece p of those four
+        if constexpr (p < 4)
+          read_piece(na, nb, std::integral_constant<int, FM + p / 2>{}, std::integral_constant<int, p % 2>{});
         if constexpr (i == NM - 1) read_piece(na, nb, std::integral_constant<int, FM - 1>{}, H1{});
       } else if constexpr (!LAST) {
         constexpr int r0 = spread_lo(i, NR, NM), r1 = spread_hi(i, NR, NM);
@@ -592,7 +594,9 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
   // (CH 16-byte chunks), read back SPI rows per instruction
   constexpr int SRB = 2 * TN, CH = SRB / 16, SPI = 64 / CH;
   constexpr int kEpiStores = F32 ? FM * FN : FM / 2 * (32 / SPI);
-  constexpr int kAfterEpi = kAhead + kEpiStores + (STG ? 0 : BLKB - BLKA);
+  // (EPI: the number of stores depends on the output's type and alignment;
+  // none may be left, which is always safe)
+  constexpr int kAfterEpi = kAhead + (EPI ? 0 : kEpiStores) + (STG ? 0 : BLKB - BLKA);
   static_assert(32 * SRB * NW <= (op_st == 0 ? SBA : SBB), "the staging fits its slot");
   using VmAfterEpi = std::integral_constant<int, (kAfterEpi < 64 ? kAfterEpi : 63)>;
   // Scale loads issued before the last step (row scales, column-scale
@@ -750,6 +754,36 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
         __builtin_amdgcn_sched_barrier(0);
       });
     }
+    if constexpr (EPI) {
+      // bias, activation and the output's type, from the accumulators: 4
+      // columns of a row per lane and store
+      const int nb = n0 + wn * TN + 4 * fg;
+      txd::f32x4 bias4[FN];
+#pragma unroll
+      for (int fn = 0; fn < FN; ++fn)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          bias4[fn][q] = a.bias && nb + 16 * fn + q < a.N ? a.bias[nb + 16 * fn + q] : 0.0f;
+      with_act(a.act, [&](auto act_tag) {
+        constexpr int ACT = decltype(act_tag)::value;
+        static_for<FM>([&](auto fm_tag) {
+          constexpr int fm = decltype(fm_tag)::value;
+          const int m = m0 + wm * TM + 16 * fm + frow;
+          static_for<FN>([&](auto fn_tag) {
+            constexpr int fn = decltype(fn_tag)::value;
+            float y[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              float v;
+              asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(v) : "a"(acc[fn][fm][q]));
+              y[q] = epi_act_t<ACT>(v * sav[fm] * sb4[fn][q] + bias4[fn][q]);
+            }
+            // (N is a multiple of 8: 4 columns are wholly in or out)
+            if (m < d.rows && nb + 16 * fn < a.N) epi_store4(a, m, nb + 16 * fn, y);
+          });
+        });
+      });
+    }
     uint8_t *stg = lds + stage_at + wave * (32 * SRB);
     // The lane's staging offsets are recomputed for each tile from an opaque
     // copy of the lane index: hoisted out of the tile loop, they would hold
@@ -764,7 +798,7 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
     const bool straddle = KTAIL && (d.nend & 7) != 0 && n0 + BN > d.nend;
     const int cols = KTAIL ? d.nend - n_st : 8;  // valid columns from n_st on
     const uint32_t coloff = n_st < d.nend && (!KTAIL || cols >= 8) ? uint32_t(n_st) * 2u + cmis : kOob;
-    if constexpr (!F32) static_for<FM / 2>([&](auto blk_tag) {
+    if constexpr (!F32 && !EPI) static_for<FM / 2>([&](auto blk_tag) {
       constexpr int blk = decltype(blk_tag)::value;
       static_for<2>([&](auto u_tag) {
         constexpr int u = decltype(u_tag)::value, fm = 2 * blk + u;
