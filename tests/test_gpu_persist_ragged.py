@@ -36,3 +36,40 @@ def test_persist_ragged_exact(tx, dev, M, N, K, layout, dtype, pad, shift):
     rest = buf.clone()
     rest[shift + ld:shift + ld + M * ld].view(M, ld)[:, :N] = 7.0
     assert (rest == 7.0).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_odd_k_recorded_without_scratch(tx, dev, dtype):
+    """An odd-K product below 1 Gi multiply-adds is recorded into a graph on a
+    stream that never ran one, allocates nothing there, and later eager calls
+    that do use scratch are right after the graph is gone."""
+    M, N, K = 333, 777, 555
+    g = torch.Generator().manual_seed(5)
+
+    def ints(*shape):
+        return torch.randint(-3, 4, shape, generator=g).float()
+
+    a, b = torch.empty(M, K, dtype=dtype, device=dev), torch.empty(N, K, dtype=dtype, device=dev)
+    out = torch.empty(M, N, dtype=dtype, device=dev)
+    x, y = ints(M, K), ints(N, K)
+    a.copy_(x), b.copy_(y)
+    tx.dot(a, b, out)  # loads the kernels
+    torch.cuda.synchronize()
+    side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    before = tx.lib.txScratchAllocations()
+    with torch.cuda.graph(graph, stream=side):
+        tx.dot(a, b, out)
+    assert tx.lib.txScratchAllocations() == before
+    for _ in range(3):
+        x, y = ints(M, K), ints(N, K)
+        a.copy_(x), b.copy_(y)
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.cpu(), (x @ y.t()).to(dtype))
+    graph.reset()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        tx.dot(a, b, out)
+    torch.cuda.synchronize()
+    assert torch.equal(out.cpu(), (x @ y.t()).to(dtype))

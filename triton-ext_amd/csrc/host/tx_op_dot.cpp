@@ -302,6 +302,15 @@ constexpr int64_t kPadMinWork = int64_t(1) << 30;
 // 777 x 555 45 us on the generic tile, 15 us with the copies; 411^3 37 -> 15.)
 constexpr int64_t kPadMinWork16 = int64_t(1) << 26;
 
+// True if a stream is recording a graph (or the runtime cannot tell): an
+// allocation made then belongs to the graph and goes with it.
+bool capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
+}
+
 // Widest source load (8, 4, 2 or 1 bytes) that divides the base address,
 // the row pitch and the row length of a padded copy's source.
 int pad_load_bytes(const void *src, int64_t ld_bytes, int64_t row_bytes) {
@@ -347,7 +356,10 @@ tx_status pad_operands(const char *pad, CodeObject co, tx_gemm_args &args, int e
 
 tx_status launch_padded(const char *base, const char *reduce, const char *pad, CodeObject co,
                         tx_gemm_args &args, int es, hipStream_t s) {
-  if (int64_t(args.M) * args.N * args.K < (es == 2 ? kPadMinWork16 : kPadMinWork)) return TX_UNSUPPORTED;
+  const int64_t work = int64_t(args.M) * args.N * args.K;
+  // Below kPadMinWork a recorded call stays on the generic tile, which needs
+  // no scratch, so that it can be recorded without a call before it.
+  if (work < kPadMinWork && (es != 2 || work < kPadMinWork16 || capturing(s))) return TX_UNSUPPORTED;
   ScratchLease ws;  // held until every launch using it is enqueued
   TX_TRY(pad_operands(pad, co, args, es, s, ws));
   return launch_fast(base, reduce, co, args, int64_t(args.K) * es, es, s, true);
