@@ -75,14 +75,17 @@ __device__ __forceinline__ constexpr int kn_swz(int k, int krb) {
   return (krb >= 256 ? ((rho << 1) ^ (rho << 2)) & 14 : rho << 1) ^ hi;
 }
 
-// s_waitcnt lgkmcnt(N) that the two fragments depend on (their values come
-// from LDS reads issued in inline asm, which the compiler does not wait for).
-template <int N>
-__device__ __forceinline__ void lgkm_wait_tie(txd::i32x4 &x) {
-  asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(x) : "n"(N));
+// ds_read_b64_tr_b16 at LDS pointer p.  The pointer is __restrict__ for the
+// alias scope that gives the read once inlined: without one the compiler puts
+// a vmcnt(0) (a drain of every operand load in flight) before this read
+// whenever an LDS-DMA load is pending.  (Never as inline asm with its wait
+// elsewhere: the compiler takes such a result as there at once, and copied
+// fragments of a tile's first step to other registers ahead of their wait.)
+typedef __attribute__((__vector_size__(4 * sizeof(short)))) short s16x4;
+__device__ __forceinline__ txd::u32x2 tr_read(const uint8_t *__restrict__ p) {
+  return __builtin_bit_cast(txd::u32x2,
+                            __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4 *)p));
 }
-// The same dependency on a wait already made (the barrier's).
-__device__ __forceinline__ void tie(txd::i32x4 &x) { asm volatile("" : "+v"(x)); }
 
 // One 16 x 16 block product: 64 bytes of K of 16-bit operands (a 16-byte
 // piece per lane), or the 128 bytes of a whole step of fp8 (two).
@@ -389,7 +392,6 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
   // 16 fn + 4 (s mod 4) .. + 3 of the wave's; half h and read r add K rows
   // 32 h + 4 r (which leave the swizzle alone).
   int bko[BKN ? FN : 1];
-  const uint32_t lds_base = uint32_t(reinterpret_cast<uintptr_t>((lds_u8 *)lds));
   if constexpr (BKN) {
     const int s16 = lane & 15, kr = 8 * fg + (s16 >> 2);
 #pragma unroll
@@ -403,17 +405,8 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
   auto read_piece = [&](int base_a, int base_b, auto f_tag, auto x_tag) {
     constexpr int f = decltype(f_tag)::value, x = decltype(x_tag)::value;
     if constexpr (BKN && f >= FM) {
-      // Inline asm: the compiler puts a vmcnt(0) (a drain of every operand
-      // load in flight) before the intrinsic form of this read whenever an
-      // LDS-DMA load is pending.  Its results are waited for explicitly:
-      // kn_wait in the K step's first half, the barrier in the second.
-      constexpr int c0 = 32 * x * KRB;
-      const uint32_t addr = lds_base + uint32_t(base_b + bko[f - FM]);
-      txd::u32x2 lo, hi;
-      asm volatile("ds_read_b64_tr_b16 %0, %2 offset:%3\n\tds_read_b64_tr_b16 %1, %2 offset:%4"
-                   : "=&v"(lo), "=&v"(hi)
-                   : "v"(addr), "i"(c0), "i"(c0 + 4 * KRB)
-                   : "memory");
+      const uint8_t *bp = lds + (base_b + bko[f - FM]) + 32 * x * KRB;
+      const txd::u32x2 lo = persist::tr_read(bp), hi = persist::tr_read(bp + 4 * KRB);
       fr[f][x] = txd::i32x4{int(lo[0]), int(lo[1]), int(hi[0]), int(hi[1])};
     } else {
       const uint8_t *Sp = lds + (f < FM ? base_a : base_b);
@@ -426,19 +419,6 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
   auto read = [&](int base_a, int base_b, auto h_tag, auto r_tag) {
     constexpr int o = decltype(r_tag)::value, f = o == 0 ? 0 : o == 1 ? FM : o <= FM ? o - 1 : o;
     read_piece(base_a, base_b, std::integral_constant<int, f>{}, h_tag);
-  };
-  // LDS operations of reads 0 .. r - 1 of a K half (BKN: two per B block).
-  constexpr auto read_ops = [](int r) constexpr { return r + (r >= 2 ? 1 : 0) + (r > FM + 1 ? r - FM - 1 : 0); };
-  // BKN: wait for the first half's B block fn before its first MFMA.  LDS
-  // operations complete in order, so at most the operations issued after B
-  // fn may be left outstanding: the rest of that half's reads and the second
-  // half's issued so far (capped at lgkmcnt's 15; extra scalar loads in
-  // flight only make the wait longer).  The asm ties the fragment to the wait.
-  auto kn_wait = [&](auto fn_tag) {
-    constexpr int fn = decltype(fn_tag)::value;
-    constexpr int after = read_ops(NR) - read_ops(fn == 0 ? 2 : FM + fn + 1) + read_ops(spread_lo(fn * FM, NR, RW));
-    constexpr int n = after > 15 ? 15 : after;
-    persist::lgkm_wait_tie<n>(fr[FM + fn][0]);
   };
   txd::f32x4 acc[FN][FM];
   // The MFMA of B block fn against A block fm on K half h (fp8: the whole
@@ -516,7 +496,6 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
       constexpr int i = decltype(I)::value;
       using Fn = std::integral_constant<int, i / FM>;
       using Fm = std::integral_constant<int, i % FM>;
-      if constexpr (BKN && i % FM == 0) kn_wait(Fn{});
       mma(H0{}, Fn{}, Fm{}, first_tag);
       __builtin_amdgcn_sched_barrier(0);
       if constexpr (C::FP8) {
@@ -534,10 +513,6 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
       __builtin_amdgcn_sched_barrier(0);
     });
     wait_and_barrier<VM>();
-    if constexpr (BKN) {
-      // the barrier's lgkmcnt(0) completed the second half's B reads
-      static_for<FN>([&](auto fn) { persist::tie(fr[FM + decltype(fn)::value][1]); });
-    }
     __builtin_amdgcn_sched_barrier(0);
     if (clear) persist::ktail_clear<NF>(fr, 1, fg, kt);
     static_for<NM>([&](auto I) {
