@@ -7,6 +7,7 @@ holds back an instruction that reads a result still on its way: on every path
 from such a read an `s_waitcnt lgkmcnt(n)` has to come first, with n at most
 the LDS operations issued after it.
 """
+import glob
 import os
 import re
 import subprocess
@@ -92,3 +93,19 @@ def test_transposing_reads_are_waited_for(tmp_path):
         bad = early_touches(ins)
         assert not bad, (name, len(bad), bad[:4])
     assert found >= 18, found  # persist_kn at three tiles, with 16-bit (4 pairs of types) and fp32 outputs (2)
+
+
+def test_no_load_is_issued_in_inline_asm():
+    """A load in inline asm stands with its wait in the same block, or not at
+    all: the compiler takes its result as there at once, may copy or reuse the
+    registers while the load is on its way, and does not count it."""
+    srcs = [p for p in glob.glob(os.path.join(REPO, "triton-ext_amd", "csrc", "**", "*"), recursive=True)
+            if p.endswith((".hip", ".h", ".cpp"))]
+    assert len(srcs) > 10
+    for p in srcs:
+        with open(p) as f:
+            text = f.read()
+        for m in re.finditer(r"\basm\b[^;]*?\((\s*\"(?:[^\"\\]|\\.)*\")+", text):
+            code = m[0]
+            if re.search(r"\b(global|buffer|flat|scratch)_load|\bds_read|\bds_load|\bs_load|_rtn", code):
+                assert "s_waitcnt" in code, (os.path.relpath(p, REPO), code)

@@ -177,7 +177,7 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
   constexpr int kLds = STG ? D * STAGE : kSlots * SBA;
   // The epilogue stages its output in the larger slot (A's if equal), whose
   // loads of the last step wait until it is done: operand op_st.
-  constexpr int op_st = BN > BM ? 1 : 0, kLastLoads = op_st == 0 ? BLKB : BLKA;
+  constexpr int op_st = BN > BM ? 1 : 0;
   constexpr bool ROWCOL = C::FP8;
   // BKN: bytes of a K row of the B tile, and K rows per 1 KiB DMA block
   constexpr int KRB = 2 * BN, RPB = 1024 / KRB, CPR = KRB / 16;
@@ -634,28 +634,23 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
     } else {
       for (int k = 1; k < KS - 1; ++k) step(std::false_type{}, VmStep{}, std::false_type{});
     }
-    // Scales load just before the last step and are waited for after it
-    // with vmcnt(kLastLoads), leaving its own loads in flight.  Loads and waits are
-    // written out: the compiler does not count the LDS-DMA loads when it
-    // places waits, so its own wait here would be vmcnt(0), a full drain of
-    // the next tile's operand loads (vector-memory operations complete in
-    // order, so vmcnt(n) with n = the operations issued since guarantees a
-    // load).  Rows past M read row M - 1 and columns past N the last four;
-    // their stores are dropped.
+    // Scales load just before the last step; the compiler's wait for them after
+    // it leaves that step's own loads in flight (vector-memory operations
+    // complete in order).  Exactly kScaleLoads of them, between scheduling
+    // barriers, since the last step's barrier counts them.  Rows past M read
+    // row M - 1 and columns past N the last four; their stores are dropped.
     float sav[FM];
     txd::f32x4 sb4[FN];  // columns 16 fn + 4 g .. + 3 of the wave's
     if constexpr (ROWCOL) {
+      typedef txd::f32x4 f32x4_a4 __attribute__((aligned(4)));
       const int nl = n0 + wn * TN + 4 * fg;
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int fm = 0; fm < FM; ++fm) {
-        const float *ps = d.sa + min(m0 + wm * TM + fm * 16 + frow, d.rows - 1);
-        asm volatile("global_load_dword %0, %1, off" : "=v"(sav[fm]) : "v"(ps) : "memory");
-      }
+      for (int fm = 0; fm < FM; ++fm) sav[fm] = d.sa[min(m0 + wm * TM + fm * 16 + frow, d.rows - 1)];
 #pragma unroll
-      for (int fn = 0; fn < FN; ++fn) {
-        const float *ps = d.sb + min(nl + 16 * fn, a.N - 4);
-        asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(sb4[fn]) : "v"(ps) : "memory");
-      }
+      for (int fn = 0; fn < FN; ++fn)
+        sb4[fn] = *reinterpret_cast<const f32x4_a4 *>(d.sb + min(nl + 16 * fn, a.N - 4));
+      __builtin_amdgcn_sched_barrier(0);
     }
     // F32: the accumulator operand through a buffer of its own (empty
     // without one), element (m, n) of row block fm and column block fn.
@@ -683,13 +678,6 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
     }
     const int stage_at = op_st == 1 ? sb : STG ? sa : sb;  // where the last step's op_st loads go
     step(std::false_type{}, VmLast{}, std::true_type{});  // the last step (KS >= 2)
-    if constexpr (ROWCOL) {
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kLastLoads) : "memory");
-#pragma unroll
-      for (int fm = 0; fm < FM; ++fm) asm volatile("" : "+v"(sav[fm]));
-#pragma unroll
-      for (int fn = 0; fn < FN; ++fn) asm volatile("" : "+v"(sb4[fn]));
-    }
     // Epilogue, per 32-row block: scale, round and stage the wave's 32 x TN
     // block (lane l: 4 columns 16 fn + 4 (l / 16) .. of row l % 16 of each 16 x
     // 16 block), then store SPI rows of SRB bytes per instruction.
