@@ -153,13 +153,24 @@ int small_persist_tile(int64_t M, int64_t N, int64_t k_bytes, int64_t cus) {
 // Before -> here: 2048^3 29.2 -> 13.2 us, 1024 x 4096 x 4096 31.4 -> 20.9, 512 x
 // 8192 x 2048 25.5 -> 12.7, 700 x 2048 x 2048 22.6 -> 10.6, 1500 x 6000 x 3072 41.2
 // -> 38.7; left to the other tile: 512 x 14336 x 4096, 1024 x 1024 x 8192.
-bool fp8_persist128(int64_t M, int64_t N, int64_t ksteps, int64_t cus) {
+// A fused epilogue costs each round 3.7 us more here (6.6 with silu or gelu),
+// 2.7 (5.9) on the other tile unsplit, so more rounds than the other needs
+// (three against two) only pay over a long K, measured with bias / with bias
+// and silu, other tile -> here: 1536 x 6144 x 1024 26.1 -> 30.0 / 31.5 -> 37.7 us,
+// 900 x 9000 x 4096 53.1 -> 54.0 / 59.6 -> 63.4, 3000 x 3000 x 8192 96.5 -> 95.6 /
+// 102.9 -> 105.1, 900 x 9000 x 14336 153.6 -> 148.7 / 160.1 -> 157.0.  With no more
+// rounds they gain like the plain product: 600 x 12000 x 1024 25.3 -> 20.8 /
+// 31.4 -> 26.7, 1024 x 4096 x 4096 41.0 -> 21.9 / 41.8 -> 24.8.
+constexpr int64_t kEpiRoundSteps = 96;
+bool fp8_persist128(int64_t M, int64_t N, int64_t ksteps, int64_t cus, bool epi) {
   const int64_t t128 = ((M + 127) / 128) * ((N + 127) / 128), tn = ((M + 255) / 256) * ((N + 127) / 128);
   int64_t splits = std::max<int64_t>(1, std::min({kMaxSplits, cus / tn, ksteps / kMinStepsPerSplit}));
   const int64_t per = (ksteps + splits - 1) / splits;
   splits = (ksteps + per - 1) / per;
-  const double here = double((t128 + cus - 1) / cus) * double(ksteps) * 0.5;
-  const double there = double((tn * splits + cus - 1) / cus) * double(per) +
+  const int64_t rounds = (t128 + cus - 1) / cus, rounds_there = (tn * splits + cus - 1) / cus;
+  if (epi && rounds > rounds_there && ksteps < kEpiRoundSteps) return false;
+  const double here = double(rounds) * double(ksteps) * 0.5;
+  const double there = double(rounds_there) * double(per) +
                        (splits > 1 ? 4.0 + double(splits) * double(M) * double(N) * 8.0 / 5e6 : 0.0);
   return here < 0.9 * there;
 }
@@ -228,7 +239,7 @@ tx_status launch_fast(const char *base, const char *reduce, CodeObject co, tx_ge
     // (the fused epilogue stores by itself, to C of any alignment)
     const bool ok = args.epi ? args.splits <= 1 && k_bytes >= 256 && k_bytes % 128 == 0 && args.N % 8 == 0
                              : persist_variant(args, k_bytes, es) != nullptr;
-    if (ok && fp8_persist128(args.M, args.N, k_bytes / 128, cus)) {
+    if (ok && fp8_persist128(args.M, args.N, k_bytes / 128, cus, args.epi != 0)) {
       std::snprintf(kname, sizeof kname, "%s_persist128", base);
       args.tiles_m = int32_t((args.M + 127) / 128);
       args.tiles_n = int32_t((args.N + 127) / 128);
