@@ -1,0 +1,67 @@
+"""The dispatch rules of the 16-bit dots and of small groups, on the CPU: each
+rule is taken from tx_op_dot.cpp and compiled by itself, for 256 CUs, and held
+to products timed on both sides on one MI355X (microseconds).  It may not pick
+a side that is more than 2% slower.
+"""
+import ctypes
+import os
+import re
+import shutil
+import subprocess
+
+import pytest
+
+SRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "triton-ext_amd", "csrc", "host",
+                   "tx_op_dot.cpp")
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    if not shutil.which("g++"):
+        pytest.skip("needs g++")
+    with open(SRC) as f:
+        text = f.read()
+    parts = re.findall(r"^constexpr int64_t (?:kMinStepsPerSplit|kMaxSplits|kSmallMaxSteps) = \d+;", text, re.M)
+    parts += [re.search(rf"^(?:bool|int) {fn}\(.*?^}}", text, re.M | re.S)[0]
+              for fn in ("persist_beats_split", "small_persist_tile")]
+    d = tmp_path_factory.mktemp("rules")
+    cpp, so = str(d / "rules.cpp"), str(d / "rules.so")
+    with open(cpp, "w") as f:
+        f.write("#include <algorithm>\n#include <cstdint>\n" + "\n".join(parts) + """
+extern "C" int edge(int64_t M, int64_t N, int64_t K) { return small_persist_tile(M, N, 2 * K, 256); }
+extern "C" int here(int64_t M, int64_t N, int64_t K, bool acc, bool kn) {
+  return persist_beats_split(M, N, (2 * K + 127) / 128, edge(M, N, K), 256, acc, kn);
+}
+""")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", cpp, "-o", so], check=True)
+    lib = ctypes.CDLL(so)
+    lib.edge.argtypes = [ctypes.c_int64] * 3
+    lib.here.argtypes = [ctypes.c_int64] * 3 + [ctypes.c_bool] * 2
+    return lib
+
+
+# M, N, K: the tile's edge, 256 x 128 tile with its split, persistent tile
+RAGGED = {
+    (1000, 1001, 2112): (64, 40.7, 12.6), (1000, 1001, 8192): (64, 50.0, 33.0), (1020, 1020, 4100): (64, 29.1, 22.7),
+    (1020, 1020, 6144): (64, 29.1, 26.2), (1020, 1020, 12288): (64, 38.4, 47.2), (1020, 1020, 16384): (64, 44.3, 61.6),
+    (1020, 1022, 12288): (64, 57.2, 47.2), (1000, 2001, 4100): (64, 57.5, 40.8), (1000, 2001, 6144): (64, 58.6, 48.8),
+    (1000, 2001, 12288): (64, 77.8, 91.0), (1020, 2044, 2112): (64, 27.6, 20.4), (1020, 2044, 4100): (64, 37.6, 40.9),
+    (1020, 2044, 8192): (64, 45.2, 63.2), (1500, 1100, 2112): (64, 24.9, 20.0), (1500, 1100, 4100): (64, 34.2, 41.1),
+    (1500, 1100, 16384): (64, 61.7, 120.3), (600, 3004, 2112): (64, 24.5, 20.2), (600, 3004, 6144): (64, 37.4, 48.3),
+    (3000, 1004, 2112): (64, 30.9, 28.6), (3000, 1004, 4100): (64, 49.1, 59.7), (1025, 2047, 2112): (64, 43.2, 28.5),
+    (1025, 2047, 4100): (64, 55.5, 58.2), (2100, 1900, 2112): (64, 31.2, 36.8), (2100, 1900, 8192): (64, 82.9, 122.3),
+    (2000, 2001, 2112): (128, 57.3, 21.6), (2000, 2001, 16384): (128, 147.9, 121.8),
+    (2040, 2044, 4100): (128, 57.6, 44.5), (2040, 2044, 16384): (128, 129.1, 123.7),
+    (1000, 801, 190): (64, None, None), (2500, 3001, 258): (128, None, None), (1000, 2001, 258): (64, None, None),
+}
+
+
+@pytest.mark.parametrize("shape", list(RAGGED))
+def test_ragged_picks_no_slower_tile(rules, shape):
+    edge, there, here = RAGGED[shape]
+    assert rules.edge(*shape) == edge
+    pick = rules.here(*shape, False, False)
+    if here is None:  # shapes of the persistent tile's GPU tests have to reach it
+        assert pick
+    else:
+        assert (there, here)[pick] <= 1.02 * min(there, here), (shape, pick)

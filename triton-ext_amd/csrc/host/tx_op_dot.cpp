@@ -139,6 +139,46 @@ const char *persist_variant(const tx_gemm_args &args, int64_t k_bytes, int es) {
 // 128-byte K steps (one short launch beats the K split and its reduce);
 // else 0 (the 256 x 128 tile with K split).
 constexpr int64_t kSmallMaxSteps = 32;
+
+// Whether the 16-bit product on persistent tiles of edge bt (128 or 64) beats
+// the 256 x 128 tile with its K split and reduce: for the ragged forms and
+// (acc) tt.dot with its accumulator, whose split always goes through planes and
+// a reduce.  One short round always does; else from estimates in us fitted to
+// about 150 products of 600 .. 3000 rows and K = 1024 .. 16384: a K step of a
+// round here (LDS-DMA delivery, the same in every round), and there a step that
+// slows as the chip fills, the planes, for N not a multiple of 4 the reduce's
+// scalar path, and (kn) the transpose of a row-major B.  256 x 128 tile -> here:
+// ragged 1020 x 1020 x 4100 29 -> 23, 1000 x 1001 x 8192 50 -> 33, left to the
+// other: 1020 x 1020 x 16384 44 -> 62, 1500 x 1100 x 4100 34 -> 41, 2100 x 1900 x
+// 8192 83 -> 122; with an accumulator 640 x 2000 x 2048 25 -> 21, 2048^2 x 16384 137
+// -> 120, left: 640 x 2000 x 4096 30 -> 33 and x 16384 57 -> 109, 3000 x 1000 x 8192
+// 65 -> 85, 2052 x 2048 x 8192 98 -> 107.
+bool persist_beats_split(int64_t M, int64_t N, int64_t steps, int64_t bt, int64_t cus, bool acc, bool kn) {
+  const int64_t rounds = (((M + bt - 1) / bt) * ((N + bt - 1) / bt) + cus - 1) / cus;
+  if (rounds == 1 && steps <= kSmallMaxSteps) return true;
+  const double mn = double(M) * double(N), n = double(rounds), k = double(steps);
+  double here;
+  if (acc) here = bt == 64 ? 8.0 + n * k * (kn ? 0.226 : 0.2) : 9.5 + n * (k * 0.38 + 1.0) * (kn ? 1.04 : 1.0);
+  else here = bt == 64 ? 5.0 + n * k * 0.225 : 4.0 + n * k * 0.455;
+  const int64_t tiles = ((M + 255) / 256) * ((N + 127) / 128);
+  int64_t splits = std::max<int64_t>(1, std::min({kMaxSplits, cus / tiles, steps / kMinStepsPerSplit}));
+  const int64_t per = (steps + splits - 1) / splits;
+  splits = (steps + per - 1) / per;
+  const double units = double(tiles * splits), s = double(splits);
+  double there = double((tiles * splits + cus - 1) / cus) * double(per) *
+                 (0.25 + 0.56 * std::min(1.0, units / double(cus)));
+  if (acc) {
+    const double kn_bytes = double(N) * k * 256.0;  // (slower past what the caches hold)
+    there += 8.0 + mn * ((8.0 * s + 8.0) / 5.5e6 + 1.5e-6);
+    if (kn) there += 2.5 + kn_bytes / (kn_bytes > 1.4e8 ? 3e6 : 5.5e6);
+  } else if (splits > 1) {
+    there += 8.0 + mn * ((8.0 * s + 2.0) / 5.5e6 + (N % 4 ? 2.4e-6 * s : 0.0));
+  } else {
+    there += 12.0;
+  }
+  return here * 1.03 < there;
+}
+
 int small_persist_tile(int64_t M, int64_t N, int64_t k_bytes, int64_t cus) {
   for (int bt : {128, 64})
     if (((M + bt - 1) / bt) * ((N + bt - 1) / bt) >= cus) return bt;
@@ -261,7 +301,9 @@ tx_status launch_fast(const char *base, const char *reduce, CodeObject co, tx_ge
     // here; 4000 x 1001 x 500, 51 there, 12 here)
     const int64_t tiles = bt ? ((args.M + bt - 1) / bt) * ((args.N + bt - 1) / bt) : 0;
     const bool even = 2 * ((tiles + cus - 1) / cus) * cus <= 3 * tiles || tiles <= cus;
-    if (bt && pv && (even || std::strcmp(pv, "_persist") == 0)) {
+    if (bt && pv &&
+        (std::strcmp(pv, "_persist") == 0 ||
+         (even && persist_beats_split(args.M, args.N, (k_bytes + 127) / 128, bt, cus, false, false)))) {
       std::snprintf(kname, sizeof kname, "%s_persist%d%s", base, bt, pv + std::strlen("_persist"));
       args.tiles_m = int32_t((args.M + bt - 1) / bt);
       args.tiles_n = int32_t((args.N + bt - 1) / bt);
