@@ -65,3 +65,43 @@ def test_ragged_picks_no_slower_tile(rules, shape):
         assert pick
     else:
         assert (there, here)[pick] <= 1.02 * min(there, here), (shape, pick)
+
+
+# tt.dot with its accumulator.  M, N, K, row-major B: edge, split, persistent
+ACC = {
+    (1000, 1000, 1024, 0): (64, 21.3, 9.3), (1000, 1000, 6144, 0): (64, 29.4, 26.1), (1000, 1000, 16384, 0): (64, 44.8, 57.7),
+    (1000, 1000, 8192, 1): (64, 40.5, 35.5), (1000, 1000, 16384, 1): (64, 59.6, 64.9), (1024, 1024, 4096, 0): (64, 27.0, 19.9),
+    (1024, 1024, 16384, 0): (64, 46.1, 58.0), (640, 2000, 2048, 0): (64, 25.4, 20.6), (640, 2000, 4096, 0): (64, 29.6, 33.0),
+    (640, 2000, 4096, 1): (64, 37.4, 35.3), (640, 2000, 16384, 0): (64, 57.2, 109.0), (640, 2000, 16384, 1): (64, 85.0, 118.5),
+    (1020, 2044, 4096, 0): (64, 36.9, 34.0), (1020, 2044, 8192, 0): (64, 49.3, 59.0), (1500, 1100, 2048, 0): (64, 27.7, 20.5),
+    (1500, 1100, 8192, 0): (64, 43.5, 58.3), (2048, 2048, 2048, 0): (128, 45.6, 24.2), (2048, 2048, 16384, 0): (128, 137.0, 120.5),
+    (2048, 2048, 16384, 1): (128, 158.0, 125.3), (2052, 2048, 2048, 0): (128, 46.0, 37.1), (2052, 2048, 4096, 0): (128, 63.7, 60.7),
+    (2052, 2048, 8192, 0): (128, 97.8, 107.4), (2052, 2048, 8192, 1): (128, 109.6, 113.2), (2052, 2048, 16384, 0): (128, 171.0, 205.1),
+    (2304, 2304, 4096, 0): (128, 69.7, 61.8), (2304, 2304, 8192, 0): (128, 107.5, 109.6), (2304, 2304, 16384, 0): (128, 187.7, 209.1),
+    (2304, 2304, 16384, 1): (128, 255.3, 219.4), (3000, 1000, 2048, 0): (64, 34.1, 27.9), (3000, 1000, 4096, 0): (64, 44.6, 46.8),
+    (3000, 1000, 4096, 1): (64, 49.6, 51.9), (3000, 1000, 16384, 1): (64, 122.5, 183.8), (1024, 1028, 2048, 0): (64, 26.4, 21.6),
+    (1024, 1028, 4096, 0): (64, 30.3, 34.4), (1024, 1028, 16384, 0): (64, 51.0, 109.5), (2048, 3072, 8192, 0): (128, 118.3, 110.7),
+    (600, 4000, 4096, 0): (64, 41.6, 46.6), (600, 4000, 4096, 1): (64, 54.9, 47.2), (600, 4000, 16384, 0): (64, 99.7, 160.5),
+    # shapes of the persistent tile's GPU tests
+    (100, 260, 64 * 21, 0): (64, None, None), (65, 264, 64 * 8, 1): (64, None, None), (129, 4100, 64 * 9, 0): (64, None, None),
+    (63, 8, 128, 1): (64, None, None), (1200, 2000, 64 * 9, 0): (64, None, None), (1200, 2000, 64 * 9, 1): (64, None, None),
+    (2047, 2044, 64 * 9, 0): (128, None, None), (2048, 2040, 64 * 9, 1): (128, None, None), (2001, 2052, 128, 0): (128, None, None),
+}
+
+
+@pytest.mark.parametrize("case", list(ACC))
+def test_accumulating_picks_no_slower_tile(rules, case):
+    M, N, K, kn = case
+    edge, there, here = ACC[case]
+    assert rules.edge(M, N, K) == edge
+    pick = rules.here(M, N, K, True, bool(kn))
+    if here is None:
+        assert pick
+    else:
+        assert (there, here)[pick] <= 1.02 * min(there, here), (case, pick)
+
+
+def test_accumulating_form_asks_the_rule():
+    with open(SRC) as f:
+        body = re.search(r"^static tx_status launch_acc_persist\(.*?^}", f.read(), re.M | re.S)[0]
+    assert "persist_beats_split(M, N, (kb + 127) / 128, bt, cus, true, kn)" in body

@@ -531,8 +531,9 @@ static int persist_kn_tile(const tx_gemm_args &args) {
 // tile too: a 256-, 128- or 64-wide tile by the same rule, K a whole number
 // (>= 2) of 64-element steps (ragged K: the 256-wide tile, N x K B only), N a
 // multiple of 4, C and D and their rows 16-byte aligned, every matrix
-// addressable with 32-bit byte offsets.  TX_UNSUPPORTED (nothing launched)
-// otherwise: too few tiles with a long K want the K split's planes.
+// addressable with 32-bit byte offsets, and on the smaller tiles only where
+// persist_beats_split expects them to.  TX_UNSUPPORTED (nothing launched)
+// otherwise: a long K wants the K split's planes.
 static tx_status launch_acc_persist(const char *pfx, tx_gemm_args args, bool kn, hipStream_t s) {
   const int64_t M = args.M, N = args.N, K = args.K, cus = cu_count(), lim = int64_t(1) << 31;
   const int64_t kb = K * 2;
@@ -543,6 +544,7 @@ static tx_status launch_acc_persist(const char *pfx, tx_gemm_args args, bool kn,
   int bt = 256;
   if (((M + 255) / 256) * ((N + 255) / 256) < cus) bt = small_persist_tile(M, N, kb, cus);
   if (!bt || (!whole && (kn || bt != 256))) return TX_UNSUPPORTED;
+  if (bt != 256 && !persist_beats_split(M, N, (kb + 127) / 128, bt, cus, true, kn)) return TX_UNSUPPORTED;
   if (kn) {
     if (!aligned(args.A, 16) || args.lda % 8 || !aligned(args.B, 16) || args.ldb % 8 || N % 8 ||
         (M - 1) * args.lda * 2 + kb + 16 >= lim || (K - 1) * args.ldb * 2 + N * 2 + 512 >= lim)
