@@ -22,13 +22,15 @@ def rules(tmp_path_factory):
     with open(SRC) as f:
         text = f.read()
     parts = re.findall(r"^constexpr int64_t (?:kMinStepsPerSplit|kMaxSplits|kSmallMaxSteps) = \d+;", text, re.M)
+    parts += re.findall(r"^constexpr int64_t kPadMinWork16 = .*;", text, re.M)
     parts += [re.search(rf"^(?:bool|int) {fn}\(.*?^}}", text, re.M | re.S)[0]
-              for fn in ("persist_beats_split", "small_persist_tile")]
+              for fn in ("persist_beats_split", "small_persist_tile", "pad16_pays")]
     d = tmp_path_factory.mktemp("rules")
     cpp, so = str(d / "rules.cpp"), str(d / "rules.so")
     with open(cpp, "w") as f:
         f.write("#include <algorithm>\n#include <cstdint>\n" + "\n".join(parts) + """
 extern "C" int edge(int64_t M, int64_t N, int64_t K) { return small_persist_tile(M, N, 2 * K, 256); }
+extern "C" int pad(int64_t M, int64_t N, int64_t K) { return pad16_pays(M, N, K); }
 extern "C" int here(int64_t M, int64_t N, int64_t K, bool acc, bool kn) {
   return persist_beats_split(M, N, (2 * K + 127) / 128, edge(M, N, K), 256, acc, kn);
 }
@@ -36,6 +38,7 @@ extern "C" int here(int64_t M, int64_t N, int64_t K, bool acc, bool kn) {
     subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", cpp, "-o", so], check=True)
     lib = ctypes.CDLL(so)
     lib.edge.argtypes = [ctypes.c_int64] * 3
+    lib.pad.argtypes = [ctypes.c_int64] * 3
     lib.here.argtypes = [ctypes.c_int64] * 3 + [ctypes.c_bool] * 2
     return lib
 
@@ -105,3 +108,23 @@ def test_accumulating_form_asks_the_rule():
     with open(SRC) as f:
         body = re.search(r"^static tx_status launch_acc_persist\(.*?^}", f.read(), re.M | re.S)[0]
     assert "persist_beats_split(M, N, (kb + 127) / 128, bt, cus, true, kn)" in body
+
+
+# odd K below 1 Gi multiply-adds.  M, N, K: generic tile, copies and fast tile
+ODD_K = {
+    (1000, 1000, 97): (12.0, 14.1), (1000, 1000, 161): (17.3, 13.8), (1500, 1500, 33): (9.5, 18.0),
+    (1500, 1500, 97): (12.4, 14.7), (1500, 1500, 161): (17.8, 15.5), (2000, 2000, 17): (9.4, 14.0),
+    (2000, 2000, 97): (13.1, 14.2), (2000, 2000, 193): (20.6, 14.6), (2100, 2100, 33): (10.8, 21.5),
+    (2100, 2100, 97): (17.8, 21.7), (2100, 2100, 129): (21.6, 22.8), (2100, 2100, 161): (24.9, 23.2),
+    (3000, 3000, 17): (17.6, 17.5), (3000, 3000, 97): (29.6, 18.3), (4000, 4000, 17): (21.5, 17.2),
+    (5000, 5000, 3): (31.8, 23.2), (256, 8192, 65): (11.4, 13.7), (256, 8192, 161): (18.3, 14.2),
+    (8192, 256, 33): (9.4, 13.5), (8192, 256, 193): (20.4, 15.1), (333, 777, 555): (45.3, 14.2),
+    (411, 411, 411): (37.7, 14.0), (64, 1024, 1025): (66.5, 15.2), (100, 100, 6801): (429.0, 20.5),
+    (4000, 17, 999): (59.6, 21.4), (1, 8192, 8193): (607.0, 106.0),
+}
+
+
+@pytest.mark.parametrize("shape", list(ODD_K))
+def test_odd_k_picks_no_slower_path(rules, shape):
+    generic, copies = ODD_K[shape]
+    assert (generic, copies)[rules.pad(*shape)] <= 1.02 * min(generic, copies)

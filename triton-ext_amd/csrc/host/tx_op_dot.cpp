@@ -352,8 +352,16 @@ tx_status launch_fast(const char *base, const char *reduce, CodeObject co, tx_ge
 // possible, and the caller takes the generic kernel.
 constexpr int64_t kPadMinWork = int64_t(1) << 30;
 // (16-bit operands, whose copies then take the small persistent tiles: 333 x
-// 777 x 555 45 us on the generic tile, 15 us with the copies; 411^3 37 -> 15.)
-constexpr int64_t kPadMinWork16 = int64_t(1) << 26;
+// 777 x 555 45 us on the generic tile, 15 us with the copies; 411^3 37 -> 15.
+// The copies are two launches, about 14 us with the product, and the generic
+// tile's time goes with K: 2000 x 2000 x 17 / 97 / 129 / 161 9.4 / 13.1 / 16.1 / 18.5 us
+// there, 14.0 / 14.2 / 14.4 / 14.4 with copies; 2100^2, in two rounds, x 129 21.6
+// there, 22.8 with copies.  Large outputs gain at any K: 4000 x 4000 x 17 21.5 ->
+// 17.2, 5000 x 5000 x 3 31.8 -> 23.2, 3000 x 3000 x 17 level.)
+constexpr int64_t kPadMinWork16 = int64_t(1) << 26, kPadMinK16 = 144, kPadMinOut16 = 9000000;
+bool pad16_pays(int64_t M, int64_t N, int64_t K) {
+  return M * N * K >= kPadMinWork16 && (K >= kPadMinK16 || M * N >= kPadMinOut16);
+}
 
 // True if a stream is recording a graph (or the runtime cannot tell): an
 // allocation made then belongs to the graph and goes with it.
@@ -412,7 +420,7 @@ tx_status launch_padded(const char *base, const char *reduce, const char *pad, C
   const int64_t work = int64_t(args.M) * args.N * args.K;
   // Below kPadMinWork a recorded call stays on the generic tile, which needs
   // no scratch, so that it can be recorded without a call before it.
-  if (work < kPadMinWork && (es != 2 || work < kPadMinWork16 || capturing(s))) return TX_UNSUPPORTED;
+  if (work < kPadMinWork && (es != 2 || !pad16_pays(args.M, args.N, args.K) || capturing(s))) return TX_UNSUPPORTED;
   ScratchLease ws;  // held until every launch using it is enqueued
   TX_TRY(pad_operands(pad, co, args, es, s, ws));
   return launch_fast(base, reduce, co, args, int64_t(args.K) * es, es, s, true);
