@@ -24,13 +24,16 @@ def rules(tmp_path_factory):
     parts = re.findall(r"^constexpr int64_t (?:kMinStepsPerSplit|kMaxSplits|kSmallMaxSteps) = \d+;", text, re.M)
     parts += re.findall(r"^constexpr int64_t kPadMinWork16 = .*;", text, re.M)
     parts += [re.search(rf"^(?:bool|int) {fn}\(.*?^}}", text, re.M | re.S)[0]
-              for fn in ("persist_beats_split", "small_persist_tile", "pad16_pays")]
+              for fn in ("persist_beats_split", "small_persist_tile", "pad16_pays", "grouped_persist128")]
     d = tmp_path_factory.mktemp("rules")
     cpp, so = str(d / "rules.cpp"), str(d / "rules.so")
     with open(cpp, "w") as f:
         f.write("#include <algorithm>\n#include <cstdint>\n" + "\n".join(parts) + """
 extern "C" int edge(int64_t M, int64_t N, int64_t K) { return small_persist_tile(M, N, 2 * K, 256); }
 extern "C" int pad(int64_t M, int64_t N, int64_t K) { return pad16_pays(M, N, K); }
+extern "C" int small_groups(int64_t G, int64_t M, int64_t N, int64_t K) {
+  return grouped_persist128(G, M, N, K, 256);
+}
 extern "C" int here(int64_t M, int64_t N, int64_t K, bool acc, bool kn) {
   return persist_beats_split(M, N, (2 * K + 127) / 128, edge(M, N, K), 256, acc, kn);
 }
@@ -39,6 +42,7 @@ extern "C" int here(int64_t M, int64_t N, int64_t K, bool acc, bool kn) {
     lib = ctypes.CDLL(so)
     lib.edge.argtypes = [ctypes.c_int64] * 3
     lib.pad.argtypes = [ctypes.c_int64] * 3
+    lib.small_groups.argtypes = [ctypes.c_int64] * 4
     lib.here.argtypes = [ctypes.c_int64] * 3 + [ctypes.c_bool] * 2
     return lib
 
@@ -128,3 +132,30 @@ ODD_K = {
 def test_odd_k_picks_no_slower_path(rules, shape):
     generic, copies = ODD_K[shape]
     assert (generic, copies)[rules.pad(*shape)] <= 1.02 * min(generic, copies)
+
+
+# grouped fp8: groups, rows each, N, K: transposed tile, persistent 128 x 256 tile
+GROUPED = {
+    (1, 100, 14336, 4096): (27.0, 29.7), (2, 100, 14336, 4096): (28.7, 30.1), (3, 100, 14336, 4096): (36.4, 34.8),
+    (4, 100, 4096, 4096): (26.8, 28.3), (8, 16, 4096, 4096): (28.9, 28.9), (8, 128, 4096, 4096): (34.5, 31.5),
+    (8, 190, 4096, 4096): (45.2, 34.3), (16, 130, 2048, 4096): (34.9, 32.6), (32, 129, 4096, 2048): (94.3, 76.9),
+    (64, 16, 2048, 4096): (139.4, 101.4), (128, 130, 512, 512): (28.3, 24.3), (1, 100, 256, 4096): (24.4, 27.3),
+    (3, 150, 256, 8192): (40.5, 46.3), (8, 64, 256, 7168): (36.7, 41.7), (8, 129, 128, 4096): (24.5, 28.1),
+    (16, 129, 136, 1024): (14.6, 15.6), (16, 20, 512, 512): (15.2, 12.9), (16, 20, 1024, 2048): (18.4, 19.7),
+    (8, 64, 2048, 4096): (26.4, 28.4), (2, 128, 16384, 2048): (21.9, 21.2), (4, 128, 8192, 1024): (17.7, 16.3),
+    (5, 150, 7168, 2048): (37.2, 34.1), (6, 128, 5120, 1536): (20.9, 19.1), (12, 100, 4096, 4096): (41.2, 38.6),
+}
+
+
+@pytest.mark.parametrize("case", list(GROUPED))
+def test_small_groups_pick_no_slower_tile(rules, case):
+    G, rows, N, K = case
+    trans, pers = GROUPED[case]
+    assert (trans, pers)[rules.small_groups(G, G * rows, N, K)] <= 1.02 * min(trans, pers)
+
+
+def test_small_groups_gpu_tests_reach_the_tile(rules):
+    for G, M, N, K in [(8, 500, 264, 256), (9, 700, 2048, 640), (512, 32000, 128, 256), (4096, 4000, 8, 256),
+                       (7, 1000, 520, 384), (64, 6400, 1000, 256), (10, 798, 1032, 640), (40, 4000, 2048, 512)]:
+        assert rules.small_groups(G, M, N, K)
+    assert not rules.small_groups(4, 4 * 192, 2048, 512)

@@ -1050,6 +1050,20 @@ static tx_status dot_scaled_mx(const void *A, tx_dtype a_type, int64_t lda, cons
 // and most m tiles with a map (1 MiB).
 constexpr int64_t kOrderMaxGroups = 512, kMapMaxTiles = 65536;
 
+// Whether groups averaging under 192 rows take the persistent 128 x 256 tile
+// rather than the transposed 256 x 128 one (8 wavefronts, a workgroup per
+// tile), whose K steps are shorter while tiles are alone on their CUs: not with
+// fewer tiles than 15/32 of the CUs (a tile at least for each group that can
+// have a row) and 8 or more K steps.  Transposed -> persistent: 8 groups x 129 rows x
+// 128 columns x K = 4096 24.5 -> 28.0 us, 1 x 100 x 14336 x 4096 (56 tiles) 27.0 -> 29.7, 2 x
+// 100 x 14336 x 4096 (112) 28.7 -> 30.1; 6 x 128 x 5120 x 1536 (120) 20.9 -> 19.1, 3 x 100 x
+// 14336 x 4096 (168) 36.4 -> 34.8, 16 x 20 x 512 x 512 (32 tiles, 4 steps) 15.1 -> 12.9.
+bool grouped_persist128(int64_t groups, int64_t M, int64_t N, int64_t K, int64_t cus) {
+  if (M >= 192 * groups) return false;
+  const int64_t mtiles = std::max((M + 127) / 128, std::min(groups, M));
+  return 32 * mtiles * ((N + 255) / 256) >= 15 * cus || K < 8 * 128;
+}
+
 // Grouped (offsets != NULL) or batched fp8 scaled dot, bf16 out: the fast
 // tile over every (problem, tile) pair in one launch (tx_grouped_args).  The
 // group sizes stay on the device: a one-workgroup scan turns the offsets
@@ -1093,14 +1107,15 @@ static tx_status dot_fp8_grouped_impl(const char *what, const void *A, tx_dtype 
   // Groups averaging under 192 rows take tiles of 128 of their rows (a 100-row
   // group wastes 28 rows of a tile, not 156) and 256 columns: on the
   // persistent kernel where it takes the operands (K a whole number (>= 2) of
-  // 128-byte steps, 16-byte aligned C rows), else on the transposed tile,
+  // 128-byte steps, 16-byte aligned C rows) and has the tiles for it
+  // (grouped_persist128), else on the transposed tile,
   // one workgroup per tile, each paying a pipeline fill and an epilogue.
   // Before -> persistent, 2048 x 4096 weights: 64 experts, 8192 / 2048 / 256
   // rows 181 / 174 / 142 -> 157 / 127 / 96 us; 32 x 4096 x 2048, 4096 rows 97
   // -> 83; 8 x 4096 x 4096, 1024 rows 42 -> 39.
   const bool pers_ok = grouped && !e.on() && K % 128 == 0 && K >= 256 && N % 8 == 0 && aligned(C, 16) &&
                        ldc % 8 == 0 && ((M - 1) * ldc + N) * 2 < (int64_t(1) << 31);
-  const bool pers128 = pers_ok && M < 192 * groups;
+  const bool pers128 = pers_ok && grouped_persist128(groups, M, N, K, cus);
   const bool trans = grouped && !e.on() && M < 192 * groups && !pers128;
   const int64_t tile_rows = trans || pers128 ? 128 : 256;
   const int64_t rt = (M + tile_rows - 1) / tile_rows;
