@@ -23,14 +23,16 @@ def rules(tmp_path_factory):
         text = f.read()
     parts = re.findall(r"^constexpr int64_t (?:kMinStepsPerSplit|kMaxSplits|kSmallMaxSteps) = \d+;", text, re.M)
     parts += re.findall(r"^constexpr int64_t kPadMinWork16 = .*;", text, re.M)
+    parts += re.findall(r"^constexpr int64_t kOrderMaxGroups = \d+;", text, re.M)
     parts += [re.search(rf"^(?:bool|int) {fn}\(.*?^}}", text, re.M | re.S)[0]
-              for fn in ("persist_beats_split", "small_persist_tile", "pad16_pays", "grouped_persist128")]
+              for fn in ("persist_beats_split", "small_persist_tile", "pad16_pays", "grouped_persist128", "grouped_dealt")]
     d = tmp_path_factory.mktemp("rules")
     cpp, so = str(d / "rules.cpp"), str(d / "rules.so")
     with open(cpp, "w") as f:
         f.write("#include <algorithm>\n#include <cstdint>\n" + "\n".join(parts) + """
 extern "C" int edge(int64_t M, int64_t N, int64_t K) { return small_persist_tile(M, N, 2 * K, 256); }
 extern "C" int pad(int64_t M, int64_t N, int64_t K) { return pad16_pays(M, N, K); }
+extern "C" int dealt(int64_t G, int64_t N, int64_t K) { return grouped_dealt(G, N, K); }
 extern "C" int small_groups(int64_t G, int64_t M, int64_t N, int64_t K) {
   return grouped_persist128(G, M, N, K, 256);
 }
@@ -42,6 +44,7 @@ extern "C" int here(int64_t M, int64_t N, int64_t K, bool acc, bool kn) {
     lib = ctypes.CDLL(so)
     lib.edge.argtypes = [ctypes.c_int64] * 3
     lib.pad.argtypes = [ctypes.c_int64] * 3
+    lib.dealt.argtypes = [ctypes.c_int64] * 3
     lib.small_groups.argtypes = [ctypes.c_int64] * 4
     lib.here.argtypes = [ctypes.c_int64] * 3 + [ctypes.c_bool] * 2
     return lib
@@ -159,3 +162,21 @@ def test_small_groups_gpu_tests_reach_the_tile(rules):
                        (7, 1000, 520, 384), (64, 6400, 1000, 256), (10, 798, 1032, 640), (40, 4000, 2048, 512)]:
         assert rules.small_groups(G, M, N, K)
     assert not rules.small_groups(4, 4 * 192, 2048, 512)
+
+
+# groups, rows each, N, K (skewed): caller's order, dealt over the XCDs
+DEALT = {
+    (64, 128, 2048, 4096): (142.3, 140.0), (128, 60, 2048, 4096): (226.4, 222.0), (128, 180, 2048, 2048): (168.7, 172.1),
+    (64, 60, 2048, 4096): (117.7, 117.5), (64, 512, 2048, 4096): (286.0, 285.4), (16, 1000, 4096, 4096): (251.6, 255.0),
+    (64, 128, 1024, 1024): (26.7, 29.2), (32, 128, 4096, 2048): (67.7, 68.6), (128, 128, 512, 512): (22.1, 24.3),
+    (128, 128, 1024, 2048): (85.8, 90.0), (16, 128, 2048, 4096): (32.0, 35.5), (256, 128, 1024, 1024): (94.7, 102.4),
+    (256, 128, 1024, 2048): (160.8, 167.2), (256, 60, 2048, 4096): (425.3, 437.7), (64, 20, 512, 512): (12.9, 14.5),
+    (192, 20, 512, 512): (21.7, 26.3), (384, 20, 1024, 2048): (168.7, 187.0), (512, 20, 512, 512): (44.7, 69.3),
+}
+
+
+@pytest.mark.parametrize("case", list(DEALT))
+def test_dealing_is_no_slower(rules, case):
+    G, rows, N, K = case
+    order, dealt = DEALT[case]
+    assert (order, dealt)[rules.dealt(G, N, K)] <= 1.025 * min(order, dealt)

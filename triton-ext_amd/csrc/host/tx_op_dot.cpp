@@ -1046,9 +1046,21 @@ static tx_status dot_scaled_mx(const void *A, tx_dtype a_type, int64_t lda, cons
   return launch(fn, unsigned(grid), 1, 256, s, &args, sizeof args, rname);
 }
 
-// Most groups whose tiles are dealt over the XCDs (kOrderMax, gemm_fp8.hip),
-// and most m tiles with a map (1 MiB).
-constexpr int64_t kOrderMaxGroups = 512, kMapMaxTiles = 65536;
+// Most m tiles with a map (1 MiB).
+constexpr int64_t kMapMaxTiles = 65536;
+
+// Whether the groups' tiles are dealt over the XCDs (gemm_fp8.hip): the prefix
+// kernel's ranking goes with the square of the groups (1.6 us at 64 of them, 3 at
+// 128, 6 at 256, 25 at 512), and what it gives is a share of the time the
+// weights take to arrive.  Caller's order -> dealt: 64 skewed experts of 2048 x 4096
+// (512 MiB), 8192 rows, three routers 135.2 -> 137.5, 136.1 -> 130.6, 155.7 -> 151.9
+// us, 128 of them, 60 rows each 226 -> 222; not for 128 x 128 rows x 512 x 512 18.3
+// -> 20.7, 256 x 128 x 1024 x 1024 94.7 -> 102.4, 16 x 128 x 2048 x 4096 32.0 -> 35.5, 512 x
+// 20 x 512 x 512 38.4 -> 63.2, 256 x 60 x 2048 x 4096 425 -> 438.
+constexpr int64_t kOrderMaxGroups = 128;  // (kOrderMax in gemm_fp8.hip)
+bool grouped_dealt(int64_t groups, int64_t N, int64_t K) {
+  return groups > 8 && groups <= kOrderMaxGroups && groups * N * K >= int64_t(1) << 29;
+}
 
 // Whether groups averaging under 192 rows take the persistent 128 x 256 tile
 // rather than the transposed 256 x 128 one (8 wavefronts, a workgroup per
@@ -1151,8 +1163,7 @@ static tx_status dot_fp8_grouped_impl(const char *what, const void *A, tx_dtype 
   hipFunction_t fn;
   if (grouped) {
     // The persistent tiles read each m tile's problem from a map after the
-    // prefix, with the groups dealt over the XCDs (the prefix kernel's G^2
-    // ranking stays cheap up to kOrderMaxGroups), where the map fits.
+    // prefix, where the map fits.
     const int64_t map_at = (groups + 1 + 3) / 4 * 4, with_map = map_at + 4 * mtiles;
     const bool map = (pers128 || (big && pers_ok)) && (prefix_ws ? with_map <= prefix_ws_ints : mtiles <= kMapMaxTiles);
     if (prefix_ws) {  // the caller's workspace (the no-allocation entry point)
@@ -1163,7 +1174,7 @@ static tx_status dot_fp8_grouped_impl(const char *what, const void *A, tx_dtype 
     }
     if (map) {
       q.tile_map = q.tile_prefix + map_at;
-      q.dealt = groups > 8 && groups <= kOrderMaxGroups;
+      q.dealt = grouped_dealt(groups, N, K);
     }
     TX_TRY(get_kernel(CodeObject::GemmFp8, "tx_gemm_fp8_grouped_prefix", &fn));
     TX_TRY(launch(fn, 1, 1, 256, s, &q, sizeof q, "tx_gemm_fp8_grouped_prefix"));

@@ -142,10 +142,12 @@ TX_KERNEL void __launch_bounds__(256) tx_gemm_fp8_epilogue(const tx_gemm_args a)
 // (tile_prefix[groups], the total, is the same either way; the entries before
 // it are then not used.)  64 skewed experts, 8192 x 2048 x 4096, 96 m tiles: the
 // product 161 us on the transposed 256 x 128 tile, 127 us on the 128 x 256
-// persistent one with its tiles dealt.  Offsets that are not nondecreasing can give more m
-// tiles than the mtiles the map has room for: the map is then not written and
+// persistent one with its tiles dealt (about 2% of it the dealing's, which is
+// for large weights only: grouped_dealt in tx_op_dot.cpp).  Offsets that are not
+// nondecreasing can give more m tiles than the mtiles the map has room for: the
+// map is then not written and
 // the product, which sees the same total, searches the prefix.
-constexpr int kOrderMax = 512;
+constexpr int kOrderMax = 128;
 TX_KERNEL void __launch_bounds__(256) tx_gemm_fp8_grouped_prefix(const tx_grouped_args q) {
   __shared__ int wave_sum[4], cnt[kOrderMax], run_cnt[kOrderMax + 8], run_of[kOrderMax + 8];
   const int t = threadIdx.x;
