@@ -363,15 +363,6 @@ bool pad16_pays(int64_t M, int64_t N, int64_t K) {
   return M * N * K >= kPadMinWork16 && (K >= kPadMinK16 || M * N >= kPadMinOut16);
 }
 
-// True if a stream is recording a graph (or the runtime cannot tell): an
-// allocation made then belongs to the graph and goes with it.
-bool capturing(hipStream_t s) {
-  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
-  (void)hipGetLastError();
-  return true;
-}
-
 // Widest source load (8, 4, 2 or 1 bytes) that divides the base address,
 // the row pitch and the row length of a padded copy's source.
 int pad_load_bytes(const void *src, int64_t ld_bytes, int64_t row_bytes) {

@@ -167,6 +167,8 @@ struct KeptScratch {
   std::atomic<std::thread::id> owner{};  // the thread holding mu (a second lease from it is an error)
   void *ptr = nullptr;
   size_t bytes = 0;
+  bool recorded = false;        // a graph that was recorded may use ptr
+  std::vector<void *> retired;  // outgrown buffers that could not be freed for it
 };
 
 struct DeviceState {
@@ -298,6 +300,23 @@ tx_status get_kernel(CodeObject co, const char *name, hipFunction_t *out) {
   return TX_SUCCESS;
 }
 
+bool capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
+}
+
+// Device memory that belongs to no graph, also while this thread records one.
+static hipError_t malloc_outside_graph(void **p, size_t bytes) {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  hipError_t e = hipThreadExchangeStreamCaptureMode(&mode);
+  if (e != hipSuccess) return e;
+  e = hipMalloc(p, bytes);
+  (void)hipThreadExchangeStreamCaptureMode(&mode);
+  return e;
+}
+
 tx_status ScratchLease::acquire(hipStream_t stream, int slot, size_t bytes) {
   DeviceState *st = nullptr;
   tx_status s = device_state(&st);
@@ -315,6 +334,7 @@ tx_status ScratchLease::acquire(hipStream_t stream, int slot, size_t bytes) {
     own_ = true;
     return TX_SUCCESS;
   }
+  const bool recording = capturing(stream);
   KeptScratch *k;
   {
     std::lock_guard<std::mutex> g(st->map_mu);
@@ -329,12 +349,14 @@ tx_status ScratchLease::acquire(hipStream_t stream, int slot, size_t bytes) {
   k->owner.store(std::this_thread::get_id(), std::memory_order_relaxed);
   lock_ = k;
   if (k->bytes < bytes) {
-    if (k->ptr && hipFreeAsync(k->ptr, stream) != hipSuccess) (void)hipGetLastError();
+    if (k->ptr && (k->recorded || recording)) k->retired.push_back(k->ptr);
+    else if (k->ptr && hipFreeAsync(k->ptr, stream) != hipSuccess) (void)hipGetLastError();
+    k->recorded = false;
     k->ptr = nullptr;
     k->bytes = 0;
     // round up so that slowly growing requests do not reallocate every call
     const size_t want = std::min(kKeptScratch, (bytes + (size_t(4) << 20) - 1) / (size_t(4) << 20) * (size_t(4) << 20));
-    hipError_t e = hipMallocAsync(&k->ptr, want, stream);
+    hipError_t e = recording ? malloc_outside_graph(&k->ptr, want) : hipMallocAsync(&k->ptr, want, stream);
     if (e != hipSuccess) {
       (void)hipGetLastError();
       k->ptr = nullptr;
@@ -343,6 +365,7 @@ tx_status ScratchLease::acquire(hipStream_t stream, int slot, size_t bytes) {
     g_scratch_allocs.fetch_add(1, std::memory_order_relaxed);
     k->bytes = want;
   }
+  if (recording) k->recorded = true;
   ptr_ = k->ptr;
   return TX_SUCCESS;
 }
@@ -366,6 +389,10 @@ void release_all_scratch() {
     for (auto &kv : st.scratch) {
       std::lock_guard<std::mutex> kg(kv.second->mu);
       if (kv.second->ptr && hipFree(kv.second->ptr) != hipSuccess) (void)hipGetLastError();
+      for (void *p : kv.second->retired)
+        if (hipFree(p) != hipSuccess) (void)hipGetLastError();
+      kv.second->retired.clear();
+      kv.second->recorded = false;
       kv.second->ptr = nullptr;
       kv.second->bytes = 0;
     }

@@ -62,6 +62,10 @@ int cu_count();
 // stream handle that is destroyed and handed out again keeps its
 // predecessor's buffer; its work must have finished, as for any reuse of
 // memory.)  txShutdown frees the kept buffers.
+// While a stream records a graph, memory allocated on it (hipMallocAsync)
+// belongs to that graph and goes with it, so a buffer that grows in a recorded
+// call is plain hipMalloc memory.  A kept buffer that a recorded call has used
+// is not freed when it is outgrown: graphs may still use it (until txShutdown).
 constexpr size_t kKeptScratch = size_t(512) << 20;
 
 class ScratchLease {
@@ -80,6 +84,9 @@ class ScratchLease {
   bool own_ = false;    // a per-call buffer, freed by the destructor
   void *lock_ = nullptr;  // the (stream, slot) buffer whose lock this lease holds
 };
+
+// True if a stream is recording a graph (or the runtime cannot tell).
+bool capturing(hipStream_t s);
 
 // Free every kept scratch buffer of every device (txShutdown).
 void release_all_scratch();
