@@ -1,7 +1,8 @@
 """The row-wise quantiser's 1024-thread rows: codes and scales bit for bit
 against the oracle, at the row lengths and counts where the kernel changes
-(K 8192 / 16384, 256 vectors, two workgroups per CU), with vectors left over
-for some threads only, and the lengths that stay on the other paths."""
+(quant_row_wide: K from 2048 fp32 / 6144 bf16 with at most a row per CU, longer
+with more rows, up to 16384), with vectors left over for some threads only, and
+the lengths that stay on the other paths."""
 import numpy as np
 import pytest
 import torch
@@ -10,7 +11,9 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("rows,K", [(1, 2056), (3, 4096), (511, 2304), (512, 2304), (5, 2048), (700, 8192),
-                                    (700, 8200), (5, 16384), (2, 16392), (2, 8191), (600, 1028), (4, 16380)])
+                                    (700, 8200), (5, 16384), (2, 16392), (2, 8191), (600, 1028), (4, 16380),
+                                    (256, 6144), (257, 6152), (256, 6136), (300, 8200), (600, 13320), (600, 10240),
+                                    (2048, 11272), (1024, 8196)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("fmt", [1, 2])
 def test_rowwise_wide_exact(tx, oracle, dev, rows, K, dtype, fmt):

@@ -74,6 +74,27 @@ tx_status quantize_mx(const void *x, tx_dtype x_type, int64_t ldx, void *q, tx_d
   return launch(fn, unsigned(grid), 1, 256, static_cast<hipStream_t>(stream), &a, sizeof a, kname);
 }
 
+// Whether a row gets 1024 threads (kWideRow in fp8_codec.hip) instead of 256:
+// from a length on that grows with the rows.  With a workgroup per CU or
+// fewer, the row's own latency counts, and 1024 threads hold it in registers in
+// fewer steps; past one (two at 256 threads) per CU the larger workgroups wait
+// for each other, and pay where 256 threads read a row twice (K > 8192) and most
+// of their own second vectors are there.  Time of a launch, 256 -> 1024
+// threads, bf16: 16 x 4096 3.16 -> 3.23 us, 256 x 4096 3.33 -> 3.50, 256 x 8192 4.06
+// -> 3.95, 256 x 16384 6.9 -> 4.8, 511 x 8192 4.7 -> 5.4, 511 x 8200 5.8 -> 5.7, 600 x
+// 12288 7.9 -> 8.3, 1024 x 14336 12.2 -> 11.7, 4096 x 8200 26.0 -> 30.9, 4096 x 11264 34.3
+// -> 33.9, 8192 x 16384 104 -> 83; fp32: 256 x 2056 3.60 -> 3.37, 256 x 8192 5.6 -> 4.2,
+// 511 x 4096 4.2 -> 4.7, 511 x 8192 5.9 -> 5.6, 600 x 9216 7.7 -> 8.0, 600 x 10240 9.6 ->
+// 8.5, 1024 x 9216 12.3 -> 12.0, 4096 x 14336 78 -> 59.
+bool quant_row_wide(bool f32, int64_t rows, int64_t K, int64_t cus) {
+  int64_t from;
+  if (rows <= cus) from = f32 ? 2048 : 6144;
+  else if (rows < 2 * cus) from = f32 ? 6144 : 8193;
+  else if (rows < (f32 ? 4 : 8) * cus) from = f32 ? 10240 : 13312;
+  else from = f32 ? 8193 : 11264;
+  return K >= from && K <= 16384;
+}
+
 tx_status quantize_rowwise(const void *x, tx_dtype x_type, int64_t ldx, void *q, tx_dtype q_type,
                            int64_t ldq, float *scales, int64_t rows, int64_t K,
                            tx_stream_t stream) {
@@ -85,11 +106,7 @@ tx_status quantize_rowwise(const void *x, tx_dtype x_type, int64_t ldx, void *q,
   const int64_t ve = x_type == TX_F32 ? 4 : 8;  // elements per 16-byte vector
   tx_quant_args a{x, static_cast<uint8_t *>(q), scales, ldx, ldq, 0, rows, K,
                   quant_vec(x, x_type, ldx, q, ldq, K, int(ve)) ? 1 : 0, 0};
-  // 1024 threads per row (kWideRow in fp8_codec.hip): rows of more vectors
-  // than 256 threads keep in registers (K > 8192), and rows of at least two
-  // per thread when there are fewer than two such workgroups per CU
-  const bool wide = a.vec && K % ve == 0 && K <= 16384 &&
-                    (K > 8192 || (K / ve > 256 && rows < 2 * int64_t(cu_count())));
+  const bool wide = a.vec && K % ve == 0 && quant_row_wide(x_type == TX_F32, rows, K, cu_count());
   std::snprintf(kname, sizeof kname, "tx_quant_row_%s%s_%s", wide ? "wide_" : "", q_name(q_type), x_name(x_type));
   hipFunction_t fn;
   TX_TRY(get_kernel(CodeObject::Fp8Codec, kname, &fn));
