@@ -18,6 +18,8 @@ SHAPES = [
     (100, 260, 64 * 21, "nk"),    # 64-wide, 5 segments of 5 steps, the last one step
     (65, 264, 64 * 8, "kn"),      # 64-wide, 2 segments of 4
     (129, 4100, 64 * 9, "nk"),    # 64-wide, 2 segments, 5 + 4 steps
+    (1200, 2000, 64 * 9, "nk"),   # 64-wide, 608 tiles: the segment sums start again for a second and third tile
+    (1200, 2000, 64 * 9, "kn"),
     (63, 8, 128, "kn"),           # one partial tile, two K steps
     (2047, 2044, 64 * 9, "nk"),   # 128-wide, one tile per CU, 2 segments
     (2048, 2040, 64 * 9, "kn"),

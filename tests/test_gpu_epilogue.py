@@ -53,13 +53,18 @@ def _check(got, ref, out, out_scale=1.0):
 
 CASES = [
     # (M, N, K, act, out, bias, path)
-    (1024, 1024, 512, "relu", "bf16", True, "256x256"),
-    (1024, 1024, 512, "gelu_tanh", "f32", True, "256x256"),
-    (1024, 1024, 512, "silu", "f16", False, "256x256"),
-    (1024, 1024, 512, "none", "e4m3fn", True, "256x256"),
-    (512, 2048, 4096, "gelu_tanh", "bf16", True, "256x128 split K"),
-    (512, 2048, 4096, "relu", "e5m2", False, "256x128 split K"),
+    (1024, 1024, 512, "relu", "bf16", True, "128x128"),
+    (1024, 1024, 512, "gelu_tanh", "f32", True, "128x128"),
+    (1024, 1024, 512, "silu", "f16", False, "128x128"),
+    (1024, 1024, 512, "none", "e4m3fn", True, "128x128"),
+    (512, 2048, 4096, "gelu_tanh", "bf16", True, "128x128"),
+    (512, 2048, 4096, "relu", "e5m2", False, "128x128"),
+    (600, 12000, 512, "silu", "bf16", True, "128x128, more tiles than CUs"),
+    # N no multiple of 8, which the 128x128 tile does not take
+    (512, 2044, 4096, "gelu_tanh", "bf16", True, "256x128 split K"),
+    (512, 2044, 4096, "relu", "e5m2", False, "256x128 split K"),
     (300, 500, 256, "silu", "f32", True, "256x128"),
+    (1000, 1020, 512, "gelu_tanh", "f16", True, "256x128"),
     (8192, 2088, 256, "relu", "e4m3fn", True, "column strip"),
     (4352, 4096, 512, "silu", "bf16", True, "256x256, more tiles than CUs"),
     (4352, 4096, 512, "gelu_tanh", "bf16", False, "256x256, more tiles than CUs"),

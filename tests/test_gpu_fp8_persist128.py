@@ -3,8 +3,11 @@
 Integer operands (-3 .. 3) and power-of-two scales: every sum and every scaled
 value is exact in fp32, so the bf16 output is its round-to-nearest-even bit for
 bit.  M and N sit at tile edges (N a multiple of 8), K from two steps (fewer
-than the ring's five) up; one tile, a tile per CU and more tiles than CUs; all
-format pairs.  C has padding that must stay as it was.
+than the ring's five) up; one tile, a tile per CU and, for a workgroup's
+second and third tile, 564 tiles (with the fused epilogue 470: its dispatch
+wants no more rounds than 256 x 128 tiles take); all format pairs.  (2049,
+2056, 512) and (1023, 4104, 1152), a few tiles past a round, are left to 256 x
+128 tiles.  C has padding that must stay as it was.
 """
 import pytest
 import torch
@@ -13,7 +16,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("M,N,K", [(65, 128, 256), (128, 136, 640), (129, 1000, 384), (700, 2040, 768),
-                                   (2047, 2048, 512), (2049, 2056, 512), (1023, 4104, 1152)])
+                                   (2047, 2048, 512), (2049, 2056, 512), (1023, 4104, 1152), (1500, 6000, 512)])
 @pytest.mark.parametrize("fa,fb", [(0, 0), (1, 1), (0, 1), (1, 0)])
 def test_fp8_persist128_exact(tx, dev, M, N, K, fa, fb):
     dt = (torch.float8_e4m3fn, torch.float8_e5m2)
@@ -30,7 +33,8 @@ def test_fp8_persist128_exact(tx, dev, M, N, K, fa, fb):
     assert (buf[M] == 7.0).all() and (buf[:, N:] == 7.0).all()
 
 
-@pytest.mark.parametrize("M,N,K", [(65, 128, 256), (129, 1000, 384), (700, 2040, 768), (2049, 2056, 512)])
+@pytest.mark.parametrize("M,N,K", [(65, 128, 256), (129, 1000, 384), (700, 2040, 768), (2049, 2056, 512),
+                                   (600, 12000, 256)])
 @pytest.mark.parametrize("bias", [False, True])
 @pytest.mark.parametrize("act", [None, "relu"])
 @pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16, torch.float16, torch.float8_e5m2])

@@ -82,10 +82,14 @@ def test_bf16_small_shapes(tx, oracle, dev, M, N, K):
     check_close(_np_bits(C), r32, r16, BF16_TOL)
 
 
-@pytest.mark.parametrize("M,N,K", [(600, 1000, 256), (300, 500, 4096), (257, 501, 2048)])
+@pytest.mark.parametrize("M,N,K", [(600, 1000, 256), (300, 500, 4096), (257, 501, 2048), (600, 1000, 120),
+                                   (2048, 2050, 256), (257, 501, 2560)])
 def test_bf16_narrow_tile_and_split_k(tx, oracle, dev, M, N, K):
-    """Fewer 256x256 tiles than CUs: 256x128 tiles, and K split into fp32
-    partial planes (8 and 4 splits here, N not a multiple of 4 in the last)."""
+    """Fewer 256x256 tiles than CUs: 64x64 tiles (N = 1000 and N = 501 with at
+    most 32 K steps); 256x128 tiles with K whole (less than two K steps, or a
+    last round of ragged 128x128 tiles that would be nearly empty) or split
+    into fp32 partial planes (16 and 10 splits of K = 4096 and 2560, N not a
+    multiple of 4 in the last)."""
     import workloads
     A, B = workloads.bf16_gemm_input(M, N, K, seed_stream=M + N)
     C = tx.dot(_t_bf16(A, dev), _t_bf16(B, dev))

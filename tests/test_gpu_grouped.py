@@ -76,11 +76,13 @@ def test_grouped_rows_outside_groups_untouched(tx, oracle, dev):
         check_close(got[r0:r1], r32, r16, FP8_TOL)
 
 
-@pytest.mark.parametrize("N,K,fa,fb", [(1000, 256, 1, 1), (2048, 512, 2, 1)])
+@pytest.mark.parametrize("N,K,fa,fb", [(1000, 256, 1, 1), (2048, 512, 2, 1), (1001, 256, 1, 1), (1000, 272, 2, 1)])
 def test_grouped_many_small_experts(tx, oracle, dev, N, K, fa, fb):
-    """64 experts of 0..200 rows (under 192 on average): the transposed tile
-    (a group's rows along the tile's 128-wide side, C stored transposed),
-    including empty groups and a ragged N."""
+    """64 experts of 0..200 rows (under 192 on average), including empty
+    groups and a ragged N: the persistent 128 x 256 tile, and, where N is no
+    multiple of 8 or K no whole number of 128-byte steps (the last two), the
+    transposed tile (a group's rows along the tile's 128-wide side, C stored
+    transposed)."""
     g = np.random.default_rng(N + K)
     sizes = list(g.integers(0, 200, 64))
     sizes[5] = sizes[40] = 0

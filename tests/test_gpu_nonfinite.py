@@ -76,11 +76,13 @@ def _dev(x, dev, dtype=None):
 
 # Shapes and the path each takes on 256 CUs: skinny (M <= 64, K % 128 == 0),
 # the persistent 256 x 256 tile (at least one tile per CU, two K steps), the
-# 256 x 128 tile unsplit (few K steps) and with K split into fp32 partials
-# summed by the reduce kernel, the zero-padded copies (odd K, >= 2^30
-# multiply-adds) and the generic kernel (odd K, small).
-PATHS = {"skinny": (16, 1000, 512), "persistent": (4096, 4096, 256), "n128": (512, 512, 256),
-         "splitk": (300, 500, 8192), "padded": (1000, 1100, 1001), "generic": (100, 200, 300)}
+# 256 x 128 tile unsplit (few K steps, N no multiple of 8) and with K split
+# into fp32 partials summed by the reduce kernel, the zero-padded copies (odd
+# K, >= 2^30 multiply-adds), the generic kernel (odd K, small), and the
+# persistent 128 x 128 tile (one tile per workgroup, and 470 tiles).
+PATHS = {"skinny": (16, 1000, 512), "persistent": (4096, 4096, 256), "n128": (512, 508, 256),
+         "splitk": (300, 500, 8192), "padded": (1000, 1100, 1001), "generic": (100, 200, 300),
+         "persist128": (512, 512, 256), "persist128_rounds": (600, 12000, 512)}
 
 
 @pytest.mark.parametrize("path", list(PATHS))
@@ -98,11 +100,13 @@ def test_fp8_dot_nonfinite(tx, oracle, dev, path, fa, fb):
             check_classes(bf16_f32(C[r]), r32[0], got_bits=C[r], ref_bits=r16[0])
 
 
-@pytest.mark.parametrize("path", ["skinny", "persistent", "generic"])
+@pytest.mark.parametrize("path", ["skinny", "persistent", "generic", "persist128", "persist128_rounds", "n128",
+                                  "splitk"])
 def test_fp8_dot_epilogue_nonfinite(tx, oracle, dev, path):
-    """The fused epilogue (bias + relu -> bf16) on the 256 x 256 tile, and
-    after the skinny / generic kernels' scaled sums: relu keeps NaN and
-    +Inf, and sends -Inf to 0."""
+    """The fused epilogue (bias + relu -> bf16) in the 256 x 256, 128 x 128
+    and 256 x 128 tiles, the K split's reduce and the skinny kernel, and after
+    the generic kernel's scaled sums: relu keeps NaN and +Inf, and sends -Inf
+    to 0."""
     M, N, K = PATHS[path]
     fa = fb = 2
     g, aq, bq, sa, sb, rows = _case(77 + M, M, N, K, fa, fb)
@@ -119,13 +123,21 @@ def test_fp8_dot_epilogue_nonfinite(tx, oracle, dev, path):
             check_classes(got[r], y)
 
 
-@pytest.mark.parametrize("persistent", [False, True])
+GROUPED = {False: ([300, 17, 1024], 384, 512), True: ([300, 0, 17, 1500, 255, 900], 8192, 512),
+           "128x256": ([40, 0, 129, 17, 128, 1, 300, 90, 60, 33], 1032, 640),
+           "128x256 whole rounds": ([100] * 40, 2048, 512), "transposed": ([40, 0, 129, 17], 300, 272)}
+
+
+@pytest.mark.parametrize("persistent", list(GROUPED))
 def test_fp8_grouped_nonfinite(tx, oracle, dev, persistent):
-    """Grouped (mixture-of-experts) dot: the per-group tile, and the
-    persistent kernel that walks every group's 256 x 256 tiles."""
+    """Grouped (mixture-of-experts) dot: the per-group tile, the persistent
+    kernel that walks every group's 256 x 256 tiles, the persistent 128 x 256
+    tile of small groups (K steps from a start of the expert's own; the column
+    parts of a last round, whose other columns run on zeros, and 320 whole
+    tiles and parts) and the transposed tile."""
     fa, fb = 2, 1
-    g = np.random.default_rng(5 + persistent)
-    sizes, N, K = ([300, 0, 17, 1500, 255, 900], 8192, 512) if persistent else ([300, 17, 1024], 384, 512)
+    g = np.random.default_rng(5 + list(GROUPED).index(persistent))
+    sizes, N, K = GROUPED[persistent]
     M = sum(sizes)
     off = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)
     aq = _codes(g, (M, K), fa)
@@ -208,3 +220,71 @@ def test_gemv_nonfinite(tx, oracle, dev, M, fmt):
     r32, r16 = oracle.gemv_fp8_dequant(x, wq, s, group=group, fmt_w=fmt)
     check_classes(bf16_f32(y), r32, got_bits=y, ref_bits=r16)
     assert np.all(np.isnan(bf16_f32(y[M - 1])))
+
+
+# 16-bit products on the persistent tiles: whole K, ragged K and N on 64- and
+# 128-wide tiles (one tile and more than one per workgroup), row-major B.
+@pytest.mark.parametrize("M,N,K,layout", [(300, 500, 256, "nk"), (129, 1003, 132, "nk"), (1000, 2001, 258, "nk"),
+                                          (2500, 3001, 258, "nk"), (300, 504, 256, "kn")])
+@pytest.mark.parametrize("out", ["same", "acc"])
+def test_dot16_nonfinite(tx, dev, M, N, K, layout, out):
+    """Infs and NaNs in a few rows of A and columns of B: every output has the
+    class that fp32 sums of the products have (the finite operands are
+    integers, so the finite outputs are exact), the ragged K's repeated
+    chunk and the columns past N add nothing to it, and with an fp32
+    accumulator (tt.dot's third operand) its own Infs and NaN come through."""
+    if out == "acc" and N % 4:
+        N += 4 - N % 4
+    g = torch.Generator().manual_seed(M + N + K)
+    a = torch.randint(-3, 4, (M, K), generator=g).float()
+    b = torch.randint(-3, 4, (N, K), generator=g).float()
+    inf, nan = float("inf"), float("nan")
+    for i, r in enumerate((0, M // 2, M - 1)):
+        a[r, (0, K - 1, K // 2)[i]] = (inf, -inf, nan)[i]
+    for i, c in enumerate((1, N // 3, N - 1)):
+        b[c, (K - 1, 3, 0)[i]] = (-inf, nan, inf)[i]
+    c = torch.zeros(M, N)
+    if out == "acc":
+        c[2, 2], c[3, 3], c[4, N - 2] = inf, -inf, nan
+    # fp64 on the CPU: the same classes, and exact for the finite ones
+    want = (a.double() @ b.double().t() + c.double()).float()
+    dt = torch.bfloat16
+    at, bt = a.to(dt).to(dev), (b if layout == "nk" else b.t().contiguous()).to(dt).to(dev)
+    if out == "acc":
+        got = tx.dot_acc(at, bt, c.to(dev), b_layout=layout).cpu()
+    else:
+        got = (tx.dot(at, bt) if layout == "nk" else tx.dot_kn(at, bt)).cpu()
+        want = want.to(dt)
+    assert torch.equal(got.isnan(), want.isnan())
+    assert torch.equal(got.nan_to_num(nan=0.0, posinf=inf, neginf=-inf), want.nan_to_num(nan=0.0, posinf=inf, neginf=-inf))
+
+
+@pytest.mark.parametrize("n,nbins,zipf", [(100_003, 1000, 0), (131072 * 256 + 5, 30000, 1.1),
+                                          (49152 * 256 + 77, 65536, 1.1), (300_000, 30000, 0)])
+def test_scatter_f32_nonfinite(tx, dev, n, nbins, zipf):
+    """fp32 scatter-add of Infs and NaNs (fp64 slots for all bins, the mixed
+    table in one window and with spilled updates, the fp32 table): a bin that
+    gets both Infs or a NaN is NaN, one Inf keeps its sign, the others hold
+    their exact integer sums; bins that were Inf or NaN before stay so."""
+    g = np.random.default_rng(nbins + n)
+    if zipf:
+        cdf = np.cumsum(np.arange(1, nbins + 1, dtype=np.float64) ** -zipf)
+        idx = np.minimum(np.searchsorted(cdf, g.random(n) * cdf[-1], side="right"), nbins - 1).astype(np.int32)
+    else:
+        idx = g.integers(0, nbins, n, dtype=np.int32)
+    val = g.integers(-3, 4, n).astype(np.float32)
+    bad = g.integers(0, n, 60)
+    val[bad] = np.where(np.arange(60) % 3 == 0, np.inf, np.where(np.arange(60) % 3 == 1, -np.inf, np.nan))
+    for i, k in enumerate((0, 1, nbins - 1)):  # a hot bin, its neighbour and the last one
+        idx[7 + i], val[7 + i] = k, (np.inf, -np.inf, np.nan)[i]
+    start = g.integers(-9, 10, nbins).astype(np.float32)
+    start[nbins // 2], start[nbins // 3] = np.inf, np.nan
+    with np.errstate(invalid="ignore"):
+        want = start + np.bincount(idx, weights=val.astype(np.float64), minlength=nbins)
+    bins = torch.from_numpy(start).to(dev)
+    tx.atomic_rmw("fadd", bins, torch.from_numpy(idx).to(dev), torch.from_numpy(val).to(dev))
+    got = bins.cpu().numpy().astype(np.float64)
+    assert np.isnan(want).any() and np.isinf(want).any()
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    fin = ~np.isnan(want)
+    assert np.array_equal(got[fin], want[fin])

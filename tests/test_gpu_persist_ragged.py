@@ -4,7 +4,9 @@ Integer operands (-3 .. 3): every fp32 sum is exact, so the output is its
 round-to-nearest-even bit for bit.  N ends 1 .. 7 columns into an 8-column
 store, rows of C have any 2-byte alignment, K is ragged (4-byte aligned rows,
 read in place) or odd (padded copies), M and N sit at tile edges; the columns
-and rows around C must stay as they were.
+and rows around C must stay as they were.  512 and 480 tiles on 256 CUs give a
+workgroup a second tile: the ragged fetch's cursor crosses to it, and stores of
+single columns come ahead of its counted waits.
 """
 import pytest
 import torch
@@ -14,7 +16,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("M,N,K,layout", [
     (63, 65, 130, "nk"), (64, 71, 128, "nk"), (129, 1003, 66 * 2, "nk"), (500, 257, 2046, "nk"),   # 64-wide
-    (1000, 801, 190, "nk"), (2001, 2047, 258, "nk"), (2048, 2041, 192, "nk"),                      # 128-wide
+    (1000, 801, 190, "nk"), (1000, 2001, 258, "nk"),              # 64-wide, the second with 512 tiles
+    (2001, 2047, 258, "nk"), (2048, 2041, 192, "nk"), (2500, 3001, 258, "nk"),  # 128-wide: 256, 256, 480 tiles
     (700, 999, 260, "kn"), (333, 777, 555, "nk"), (411, 1237, 411, "kn"),                          # copies first
     (4097, 4093, 136, "nk")])                                                                      # 256-wide
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
