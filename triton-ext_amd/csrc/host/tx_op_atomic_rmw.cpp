@@ -9,7 +9,6 @@
 #include <algorithm>
 #include <climits>
 #include <cstdio>
-#include <cstring>
 
 #include "tx_kernel_args.h"
 #include "tx_ops.h"
@@ -23,8 +22,12 @@ constexpr int64_t kWinStep = 3 * kAggStep;  // windowed kernel: its pipelined lo
 constexpr int64_t kDirectSlots = 36864;  // bins per LDS window
 constexpr int64_t kMaxWindows = 4;       // beyond this the hash-table kernel is used
 // Spill buffer of the windowed kernel's one-pass path: records per
-// wavefront region (16 wavefronts per workgroup), and the chunk of records
-// per workgroup of the second launch that folds them into the bins.
+// wavefront region (16 wavefronts per workgroup; what does not fit goes to
+// global atomics), and the chunk of records per workgroup of the second launch
+// that folds them into the bins.  64 Mi Zipf(1.1) updates over 65,536 bins leave
+// 453 +- 21 of a wavefront's outside a 36,864-bin window and 500 +- 22 outside
+// fp32's mixed one of 34,816 bins, where more than a quarter of the wavefronts
+// fill their region.
 constexpr int64_t kSpillWave = 512;
 constexpr int64_t kSpillChunk = 3 * kWinStep;
 

@@ -694,10 +694,10 @@ constexpr int RowRegs = XT == 0 ? 8 : 4;
 // that fit are read once into registers, other rows take a pass for amax
 // and a second pass (from cache) for the codes.
 // Wide variant, 1024 threads per row of up to 2 (bf16) or 4 (fp32) vectors
-// each (K <= 16384): rows too long for the registers above, which were read
-// twice, and few rows, whose 256-thread workgroups leave the chip idle.
-// bf16 512 x 14336 8.8 -> 7.7 us, 4096 x 14336 45 -> 42, 8192 x 16384 103 ->
-// 84; fp32 4096 x 14336 88 -> 62, 8192 x 16384 184 -> 130.
+// each (K <= 16384), always in registers: rows too long for the registers
+// above, which are read twice there, and few rows, whose own latency counts
+// (quant_row_wide in tx_op_quant.cpp says from where on, with the times).  bf16
+// 4096 x 14336 43 -> 37 us, 8192 x 16384 104 -> 83; fp32 4096 x 14336 78 -> 59.
 constexpr int kWideRow = 1024;
 template <int XT>
 constexpr int kWideRegs = XT == 0 ? 4 : 2;
@@ -738,7 +738,7 @@ __device__ __forceinline__ void quant_row(const tx_quant_args &a) {
     }
     return;
   }
-  for (int64_t r = blockIdx.x; r < a.rows; r += gridDim.x) {
+  if constexpr (NB == kBlock) for (int64_t r = blockIdx.x; r < a.rows; r += gridDim.x) {
     const uint8_t *xrow = static_cast<const uint8_t *>(a.x) + r * a.ldx * (XT == 0 ? 4 : 2);
     uint8_t *qrow = a.q + r * a.ldq;
     const int64_t nvec = a.vec ? a.K / VE : 0;

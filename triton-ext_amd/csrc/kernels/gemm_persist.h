@@ -20,9 +20,9 @@
 // instruction and sum twice the K, do the same work on less: register-only
 // loops on N(0,1) operands sustain 2025 against 1765 TFLOP/s (bf16) and 4360
 // against 3970 (fp8).  In this kernel (32 x 32 -> 16 x 16, same box): fp16
-// 4096^3 row-major B 110 -> 107 us (clock 1.75 -> 2.00 GHz, MFMA busy 64 ->
+// 4096^3 row-major B 107 -> 102 us (clock 1.75 -> 2.00 GHz, MFMA busy 64 ->
 // 60%), bf16 8192^3 764 -> 721 us, 2048^3 (128 x 128) 22.8 -> 21.6 us, fp8
-// 8192^3 371 -> 359 us.  Without the LDS-DMA stream (timing only) these take
+// 8192^3 370 -> 361 us.  Without the LDS-DMA stream (timing only) these take
 // 93, 628, 19.5 and 300 us: what binds them now is that stream's power and
 // its delivery, not MFMA issue (staggering reads and loads, or forcing the
 // accumulators in place, moves nothing beyond 1%).
@@ -44,14 +44,13 @@
 // where B, two steps ahead, did not (8192^3 fp8 from HBM-resident inputs:
 // 2530 -> 2290 cycles per K step; 2146 with cached inputs either way).
 //
-// Epilogue: the scales load just before the tile's last K step, whose A
-// loads of step s+3 are deferred so that their LDS slot stages the output:
-// per 32 x 32 block the accumulators are scaled, rounded to bf16 / fp16
-// (RNE), and lanes l and l + 32 exchange halves (v_permlane32_swap); each
-// wave writes its 32 x BN / 2 block to its own quarter of that slot, reads
+// Epilogue: the scales load just before the tile's last K step, whose loads of
+// one operand (A; of 128 x 256 tiles B) are deferred so that their LDS slot
+// stages the output: per 32 rows of 16 x 16 blocks the accumulators are scaled
+// and rounded to bf16 / fp16 (RNE), a lane's 4 columns of a row 8 bytes in LDS;
+// each wave writes its 32 x BN / 2 block to its own quarter of that slot, reads
 // back whole rows (BN = 256: 4 of 256 bytes) per instruction and stores them
-// through a buffer
-// resource for C (stores past M / N are dropped).  OUT_F32 (tt.dot with its
+// through a buffer resource for C (stores past M / N are dropped).  OUT_F32 (tt.dot with its
 // accumulator operand): D = A.B + C in fp32 is written straight from the
 // accumulators, C's loads for the first row blocks issued before the last K
 // step.  EPI: the fp8 dot's fused epilogue, likewise from the accumulators.  The first K step of each
@@ -206,7 +205,6 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
   constexpr int ES = C::FP8 ? 1 : 2;
   const uint32_t kb_end = uint32_t(a.K) * ES;
   const int KS = int(KTAIL ? (kb_end + kStep - 1) / kStep : kb_end / kStep);  // K steps per tile (>= 2)
-  const int S = T * KS;                // steps of the workgroup
   const uint32_t lda_b = uint32_t(a.lda) * ES, ldb_b = uint32_t(a.ldb) * ES;
 
   // Per-lane DMA offsets within a tile: row * ld + chunk for the wave's
@@ -600,7 +598,8 @@ __device__ __forceinline__ void gemm_persist(const tx_gemm_args &a, const tx_gro
     // C as a buffer: a store whose row or column block lies past M / N gets
     // an offset past the range and is dropped (N is a multiple of 8, so a
     // 16-byte column block is wholly in or out).  KTAIL: rows of C may have
-    // any alignment; the buffer starts at the 16-byte boundary below C.
+    // any alignment; the buffer starts at the 16-byte boundary below C; N may
+    // be any, and a block that N cuts is stored column by column.
     const uint32_t cmis = KTAIL ? uint32_t(reinterpret_cast<uintptr_t>(d.out) & 15u) : 0u;
     const __amdgpu_buffer_rsrc_t crs =
         make_rsrc(d.out - cmis, uint32_t((int64_t(d.rows - 1) * a.ldc + a.N) * (F32 ? 4 : 2)) + cmis);

@@ -426,7 +426,8 @@ struct Scatter {
 
   // Picks the workgroup's hot keys (HotKeys) from the first 4 x kBlock
   // updates of its chunk; on return every lane holds the same set, with
-  // zeroed sums, and `blocks` (if given) counts the sample per kWinBlock bins.  Needs the whole workgroup; ends with a barrier.
+  // zeroed sums, and `blocks` (if given) counts the sample per kWinBlock bins.
+  // Needs the whole workgroup; ends with a barrier.
   static __device__ __forceinline__ void sample_hot(const tx_scatter_args &a, uint32_t lo, uint32_t nb, int64_t begin,
                                     int64_t end, bool vec, uint32_t *aux, HotKeys<OP> &hot,
                                     uint32_t *blocks = nullptr) {
