@@ -114,7 +114,7 @@ def test_accumulating_picks_no_slower_tile(rules, case):
 def test_accumulating_form_asks_the_rule():
     with open(SRC) as f:
         body = re.search(r"^static tx_status launch_acc_persist\(.*?^}", f.read(), re.M | re.S)[0]
-    assert "persist_beats_split(M, N, (kb + 127) / 128, bt, cus, true, kn)" in body
+    assert "!any_k && !persist_beats_split(M, N, (kb + 127) / 128, bt, cus, true, kn)" in body
 
 
 # odd K below 1 Gi multiply-adds.  M, N, K: generic tile, copies and fast tile

@@ -530,10 +530,10 @@ static int persist_kn_tile(const tx_gemm_args &args) {
 // tile too: a 256-, 128- or 64-wide tile by the same rule, K a whole number
 // (>= 2) of 64-element steps (ragged K: the 256-wide tile, N x K B only), N a
 // multiple of 4, C and D and their rows 16-byte aligned, every matrix
-// addressable with 32-bit byte offsets, and on the smaller tiles only where
-// persist_beats_split expects them to.  TX_UNSUPPORTED (nothing launched)
-// otherwise: a long K wants the K split's planes.
-static tx_status launch_acc_persist(const char *pfx, tx_gemm_args args, bool kn, hipStream_t s) {
+// addressable with 32-bit byte offsets, and on the smaller tiles (unless
+// any_k) only where persist_beats_split expects them to.  TX_UNSUPPORTED
+// (nothing launched) otherwise: a long K wants the K split's planes.
+static tx_status launch_acc_persist(const char *pfx, tx_gemm_args args, bool kn, hipStream_t s, bool any_k) {
   const int64_t M = args.M, N = args.N, K = args.K, cus = cu_count(), lim = int64_t(1) << 31;
   const int64_t kb = K * 2;
   if (N % 4 || kb < 256 || !aligned(args.C, 16) || args.ldc % 4 || (M - 1) * args.ldc * 4 + N * 4 >= lim ||
@@ -543,7 +543,7 @@ static tx_status launch_acc_persist(const char *pfx, tx_gemm_args args, bool kn,
   int bt = 256;
   if (((M + 255) / 256) * ((N + 255) / 256) < cus) bt = small_persist_tile(M, N, kb, cus);
   if (!bt || (!whole && (kn || bt != 256))) return TX_UNSUPPORTED;
-  if (bt != 256 && !persist_beats_split(M, N, (kb + 127) / 128, bt, cus, true, kn)) return TX_UNSUPPORTED;
+  if (bt != 256 && !any_k && !persist_beats_split(M, N, (kb + 127) / 128, bt, cus, true, kn)) return TX_UNSUPPORTED;
   if (kn) {
     if (!aligned(args.A, 16) || args.lda % 8 || !aligned(args.B, 16) || args.ldb % 8 || N % 8 ||
         (M - 1) * args.lda * 2 + kb + 16 >= lim || (K - 1) * args.ldb * 2 + N * 2 + 512 >= lim)
@@ -813,24 +813,37 @@ static tx_status dot_acc(const void *A, tx_dtype a_type, int64_t lda, const floa
   else std::snprintf(base, sizeof base, "tx_gemm_%s_fast", a_type == TX_BF16 ? "bf16" : "f16");
   const char *reduce = fp8 ? "tx_gemm_fp8_splitk_reduce" : "tx_gemm_bf16_splitk_reduce";
   if (K == 0) return launch_acc(base, reduce, co, args, 0, s);
-  if (b16 && d_type == TX_F32) {
-    // one launch of the persistent tile (nothing launched: TX_UNSUPPORTED)
-    const tx_status st = launch_acc_persist(a_type == TX_BF16 ? "bf16" : "f16", args, kn, s);
-    if (st != TX_UNSUPPORTED) return st;
-    clear_error();
+  const tx_gemm_args in_place = args;
+  auto one_launch = [&](bool any_k) {
+    return b16 && d_type == TX_F32 ? launch_acc_persist(a_type == TX_BF16 ? "bf16" : "f16", in_place, kn, s, any_k)
+                                   : TX_UNSUPPORTED;
+  };
+  // one launch of the persistent tile (nothing launched: TX_UNSUPPORTED)
+  tx_status st = one_launch(false);
+  if (st != TX_UNSUPPORTED) return st;
+  clear_error();
+  auto with_planes = [&]() -> tx_status {
+    ScratchLease ws;  // operand copies (slot 0), held until the product is enqueued
+    if (kn) {
+      TX_TRY(transpose_kn(what, args, s, ws));
+    } else if (!fast_ok(A, lda * es, B, ldb * es, K * es, M, N) &&
+               !(b16 && fast16_ragged_ok(A, lda * es, B, ldb * es, K * es, M, N))) {
+      const tx_status pad =
+          pad_operands(fp8 ? "tx_gemm_fp8_pad_rows" : "tx_gemm_bf16_pad_rows", co, args, es, s, ws);
+      if (pad == TX_UNSUPPORTED)
+        return fail(TX_UNSUPPORTED, "%s: operands too large for the zero-padded copies", what);
+      TX_TRY(pad);
+    }
+    return launch_acc(base, reduce, co, args, int64_t(args.K) * es, s);
+  };
+  st = with_planes();
+  if (st == TX_GENERIC_FAILURE) {
+    // no scratch to be had: the one launch at any K, where it takes the operands
+    const tx_status one = one_launch(true);
+    if (one == TX_SUCCESS) clear_error();
+    if (one != TX_UNSUPPORTED) return one;
   }
-  ScratchLease ws;  // operand copies (slot 0), held until the product is enqueued
-  if (kn) {
-    TX_TRY(transpose_kn(what, args, s, ws));
-  } else if (!fast_ok(A, lda * es, B, ldb * es, K * es, M, N) &&
-             !(b16 && fast16_ragged_ok(A, lda * es, B, ldb * es, K * es, M, N))) {
-    const tx_status st =
-        pad_operands(fp8 ? "tx_gemm_fp8_pad_rows" : "tx_gemm_bf16_pad_rows", co, args, es, s, ws);
-    if (st == TX_UNSUPPORTED)
-      return fail(TX_UNSUPPORTED, "%s: operands too large for the zero-padded copies", what);
-    TX_TRY(st);
-  }
-  return launch_acc(base, reduce, co, args, int64_t(args.K) * es, s);
+  return st;
 }
 
 // The fused epilogue's options (bias, tx_activation, output type and, for
